@@ -100,14 +100,14 @@ std::atomic<Device*> g_dev[64] = {};
 enum EnvKey {
   kEnvGemv1, kEnvGemv1p, kEnvGemvCfg, kEnvGemvWavesPerCu, kEnvGemvRows, kEnvSplitK, kEnvMmq2, kEnvMmq,
   kEnvMmq4Bn, kEnvMmq1, kEnvMmqXcd, kEnvMoeGemv, kEnvMoeMmq, kEnvMoeBm, kEnvMoeSplitK, kEnvMoeGrouped, kEnvGroupedP,
-  kEnvGroupedWgs, kEnvStreamK, kEnvGemvm, kEnvMmq6, kEnvMmq8, kEnvMoeTails, kEnvFfnPair, kEnvQkvSeparate, kEnvAttnOSeparate, kEnvCount
+  kEnvGroupedWgs, kEnvStreamK, kEnvGemvm, kEnvMmq6, kEnvMmq8, kEnvMoeTails, kEnvFfnPair, kEnvQkvSeparate, kEnvAttnOSeparate, kEnvPrefillAttn, kEnvCount
 };
 const char* const kEnvNames[kEnvCount] = {
     "QMM_GEMV1", "QMM_GEMV1P", "QMM_GEMV_CFG", "QMM_GEMV_WAVES_PER_CU", "QMM_GEMV_ROWS", "QMM_SPLITK",
     "QMM_MMQ2", "QMM_MMQ", "QMM_MMQ4_BN", "QMM_MMQ1", "QMM_MMQ_XCD", "QMM_MOE_GEMV", "QMM_MOE_MMQ",
     "QMM_MOE_BM", "QMM_MOE_SPLITK", "QMM_MOE_GROUPED", "QMM_GROUPED_P", "QMM_GROUPED_WGS",
     "QMM_STREAMK", "QMM_GEMVM", "QMM_MMQ6", "QMM_MMQ8", "QMM_MOE_TAILS", "QMM_FFN_SEPARATE", "QMM_QKV_SEPARATE",
-    "QMM_ATTN_O_SEPARATE"};
+    "QMM_ATTN_O_SEPARATE", "QMM_PREFILL_ATTN"};
 
 struct Tuning {
   int w = 0, r = 0, u = 0, waves_per_cu = 0, gemv1 = 1, gemv1p = -1;
@@ -2102,6 +2102,23 @@ int qmm_rope_kv_append_n(float* q, float* k, const float* v, int64_t ldq, int64_
   return QMM_OK;
 }
 
+// Whether a prompt's causal attention runs on 32-column MFMA tiles
+// (qmm_prefill_attn_tile_*) or one workgroup per row (qmm_prefill_attention_*).
+// A tile's workgroup needs ~5 us per 128 positions (head_dim 128) however few of
+// its columns are used; a row's needs n times 0.02 / 0.04 / 0.075 us for 1 / 4 / 8
+// heads a kv head, and beyond two workgroups a CU rows also queue. Measured, rows
+// against tiles, us: 32 / 8 heads of 128, 64 rows from position 0 9.6 / 10.3, 128
+// rows 18.8 / 11.5, 1999 rows 1650 / 308; 64 rows from 500 42 / 32; 16 / 16 heads,
+// 128 rows 11.9 / 11.1; 32 / 4 heads, 12 rows 9.8 / 9.9, 32 rows 11.1 / 9.9, and 2
+// rows from 500 42 / 26; 8 / 2 heads of 64, 128 rows 7.6 / 8.0, 256 rows 14.2 / 11.1.
+// (QMM_PREFILL_ATTN=rows|tiles forces one for the sizes both take.)
+static bool prefill_attn_tiles(int64_t first, int64_t count, int heads, int kv_heads, int head_dim) {
+  if (head_dim > 128) return false;  // 256: the tile's sums and V rows exceed the registers
+  if (const char* e = env(kEnvPrefillAttn)) return strcmp(e, "rows") != 0;
+  if (heads / kv_heads > 4) return count * heads >= 512 || first + count >= 512;
+  return count * heads >= 2048;
+}
+
 int qmm_prefill_attention(const float* q, int64_t ldq, const float* kcache, const float* vcache, int64_t first,
                           int64_t count, float* out, int64_t ldo, int heads, int kv_heads, int head_dim, int max_seq,
                           float scale, void* stream) {
@@ -2118,11 +2135,19 @@ int qmm_prefill_attention(const float* q, int64_t ldq, const float* kcache, cons
   const int G = heads / kv_heads;
   const int gt = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
   char name[64];
-  snprintf(name, sizeof(name), "qmm_prefill_attention_d%d_g%d", head_dim / 64, gt);
   long long a = ldq, o = ldo;
-  int f = (int)first;
-  void* args[] = {&q, &a, &kcache, &vcache, &f, &out, &o, &heads, &kv_heads, &max_seq, &scale};
+  int f = (int)first, c = (int)count;
   hipFunction_t fn;
+  if (prefill_attn_tiles(first, count, heads, kv_heads, head_dim)) {
+    snprintf(name, sizeof(name), "qmm_prefill_attn_tile_d%d", head_dim / 32);
+    void* args[] = {&q, &a, &kcache, &vcache, &f, &c, &out, &o, &heads, &kv_heads, &max_seq, &scale};
+    QMM_TRY(kernel(d, name, &fn));
+    QMM_HIP(hipModuleLaunchKernel(fn, (unsigned)kv_heads, ceil_div(count, 32 / G), 1, 256, 1, 1, 0,
+                                  (hipStream_t)stream, args, nullptr));
+    return QMM_OK;
+  }
+  snprintf(name, sizeof(name), "qmm_prefill_attention_d%d_g%d", head_dim / 64, gt);
+  void* args[] = {&q, &a, &kcache, &vcache, &f, &out, &o, &heads, &kv_heads, &max_seq, &scale};
   QMM_TRY(kernel(d, name, &fn));
   QMM_HIP(hipModuleLaunchKernel(fn, (unsigned)kv_heads, (unsigned)count, 1, 256, 1, 1, 0, (hipStream_t)stream, args,
                                 nullptr));
@@ -2181,16 +2206,23 @@ int qmm_prefill_attention_o(const float* q, int64_t ldq, const float* kcache, co
   const Planes pl = mmq_planes(wo->dtype, count, H);
   const int gt = G <= 1 ? 1 : G <= 2 ? 2 : G <= 4 ? 4 : 8;
   char name[64];
-  snprintf(name, sizeof(name), "qmm_prefill_attention_planes_d%d_g%d", head_dim / 64, gt);
   long long a = ldq;
-  int f = (int)first, kq = (int)H;
+  int f = (int)first, c = (int)count, kq = (int)H;
   void* q8 = b + pl.q8;
   void* dd = b + pl.d;
   void* ss = b + pl.s;
-  void* args[] = {&q, &a, &kcache, &vcache, &f, &q8, &dd, &ss, &kq, &heads, &kv_heads, &max_seq, &scale};
   hipFunction_t fn;
-  QMM_TRY(kernel(d, name, &fn));
-  QMM_HIP(hipModuleLaunchKernel(fn, (unsigned)kv_heads, (unsigned)count, 1, 256, 1, 1, 0, s, args, nullptr));
+  if (prefill_attn_tiles(first, count, heads, kv_heads, head_dim)) {
+    snprintf(name, sizeof(name), "qmm_prefill_attn_tile_planes_d%d", head_dim / 32);
+    void* args[] = {&q, &a, &kcache, &vcache, &f, &c, &q8, &dd, &ss, &kq, &heads, &kv_heads, &max_seq, &scale};
+    QMM_TRY(kernel(d, name, &fn));
+    QMM_HIP(hipModuleLaunchKernel(fn, (unsigned)kv_heads, ceil_div(count, 32 / G), 1, 256, 1, 1, 0, s, args, nullptr));
+  } else {
+    snprintf(name, sizeof(name), "qmm_prefill_attention_planes_d%d_g%d", head_dim / 64, gt);
+    void* args[] = {&q, &a, &kcache, &vcache, &f, &q8, &dd, &ss, &kq, &heads, &kv_heads, &max_seq, &scale};
+    QMM_TRY(kernel(d, name, &fn));
+    QMM_HIP(hipModuleLaunchKernel(fn, (unsigned)kv_heads, (unsigned)count, 1, 256, 1, 1, 0, s, args, nullptr));
+  }
   // the GEMM as matmul_targets runs it: planes first, split partials in the rest
   return gemm(d, wo, b, count, x, ldx, nullptr, s, 1, (float*)(b + pl.total), ws_bytes - pl.total);
 }

@@ -10,4 +10,5 @@
 #include "qmm_moe_kernels.h"
 #include "qmm_gemvm_kernels.h"
 #include "qmm_decode_kernels.h"
+#include "qmm_prefill_attn_kernels.h"
 #include "qmm_calib_kernels.h"
