@@ -400,35 +400,19 @@ int qmm_qtensor_quantize(int dtype, int64_t n, int64_t k, const float* w, void* 
   QMM_TRY(alloc_tensor(dtype, n, k, &t));
   const int fmt = fmt_of(dtype);
   long long nblocks = n * (k / qmm_block_size(dtype));
-  void* ggml = t->data;
   int rc = QMM_OK;
-  if (fmt != kFmtQ4K) {
-    hipError_t e = hipMalloc(&ggml, t->bytes);
-    if (e != hipSuccess) {
-      qmm_qtensor_free(t);
-      return fail(QMM_ERR_OOM, "hipMalloc(staging %zu): %s", t->bytes, hipGetErrorString(e));
-    }
+  // (Q8_0: the limit of the 32-bit value count that this call has always had)
+  if (fmt == kFmtQ80 && (long long)(int)(n * k) != n * k) rc = fail(QMM_ERR_INVALID, "Q8_0 tensor too large");
+  if (rc == QMM_OK) {
+    // every quantizer writes the device layout; 8, 16 and 8 lanes per block
+    const char* name = fmt == kFmtQ4K ? "qmm_quantize_q4k_w" : fmt == kFmtQ6K ? "qmm_quantize_q6k_w" : "qmm_quantize_q8_0_w";
+    void* data = t->data;
+    void* args[] = {&w, &data, &nblocks};
+    rc = launch(d, name, ceil_div(nblocks * (fmt == kFmtQ6K ? 16 : 8), 256), 256, 0, s, args);
   }
-  if (fmt == kFmtQ80) {
-    // Q8_0 weights use the same from_float as Q8_0 activations: treat the
-    // matrix as one row of n*k values.
-    long long ld = 0;
-    int kk = (int)(n * k), one = 1;
-    if ((long long)kk != n * k) rc = fail(QMM_ERR_INVALID, "Q8_0 tensor too large");
-    const float* x = w;
-    void* args[] = {&x, &ld, &ggml, &kk, &one};
-    if (rc == QMM_OK) rc = launch(d, "qmm_quantize_q8_0", ceil_div(nblocks * 8, 256), 256, 0, s, args);
-  } else {
-    const float* x = w;
-    void* args[] = {&x, &ggml, &nblocks};
-    rc = launch(d, fmt == kFmtQ4K ? "qmm_quantize_q4k_w" : "qmm_quantize_q6k_w", ceil_div(nblocks, 64), 64,
-                0, s, args);
-  }
-  if (rc == QMM_OK && fmt != kFmtQ4K) rc = ggml_to_dev(d, t, ggml, s);
-  if (fmt != kFmtQ4K) {
-    hipError_t e = hipStreamSynchronize(s);
-    if (rc == QMM_OK && e != hipSuccess) rc = fail(QMM_ERR_HIP, "sync: %s", hipGetErrorString(e));
-    (void)hipFree(ggml);
+  if (rc == QMM_OK && fmt != kFmtQ4K) {  // these two return with the tensor ready, as they always have
+    const hipError_t e = hipStreamSynchronize(s);
+    if (e != hipSuccess) rc = fail(QMM_ERR_HIP, "sync: %s", hipGetErrorString(e));
   }
   if (rc != QMM_OK) {
     qmm_qtensor_free(t);

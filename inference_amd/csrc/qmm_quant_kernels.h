@@ -89,12 +89,9 @@ __device__ __forceinline__ void q8k_block(const float* __restrict__ xs, uint8_t*
 //   d = amax / 127, q = round(x * (1/d)) (0 when d == 0), d stored as f16.
 // Writes GGML 34-byte blocks.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void q80_block(const float* __restrict__ xs, uint8_t* __restrict__ blk,
-                                          int l, bool valid) {
+// Lane l (of the block's 8): its four quants; *dh the block's f16 scale.
+__device__ __forceinline__ uint32_t q80_lane(const float (&e)[4], uint16_t* dh) {
 #pragma clang fp contract(off)
-  float e[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) e[j] = valid ? xs[4 * l + j] : 0.0f;
   float amax = 0.0f;
 #pragma unroll
   for (int j = 0; j < 4; ++j) amax = fmaxf(amax, fabsf(e[j]));
@@ -103,7 +100,7 @@ __device__ __forceinline__ void q80_block(const float* __restrict__ xs, uint8_t*
   amax = fmaxf(amax, dpp_f<0x141>(amax));
   const float d = amax / 127.0f;
   const float id = d != 0.0f ? 1.0f / d : 0.0f;
-  if (!valid) return;
+  *dh = f2h(d);
   uint32_t q4 = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -111,14 +108,33 @@ __device__ __forceinline__ void q80_block(const float* __restrict__ xs, uint8_t*
     r = fminf(fmaxf(r, -128.0f), 127.0f);
     q4 |= (uint32_t)((int)r & 0xff) << (8 * j);
   }
+  return q4;
+}
+
+__device__ __forceinline__ void q80_block(const float* __restrict__ xs, uint8_t* __restrict__ blk,
+                                          int l, bool valid) {
+  float e[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) e[j] = valid ? xs[4 * l + j] : 0.0f;
+  uint16_t d;
+  const uint32_t q4 = q80_lane(e, &d);
+  if (!valid) return;
   uint16_t* p = reinterpret_cast<uint16_t*>(blk);
-  if (l == 0) p[0] = f2h(d);
+  if (l == 0) p[0] = d;
   p[1 + 2 * l] = (uint16_t)(q4 & 0xffff);
   p[2 + 2 * l] = (uint16_t)(q4 >> 16);
 }
 
 // ---------------------------------------------------------------------------
-// Q4_K weight quantizer (one thread per 256-element super-block).
+// Weight quantizers: one lane per sub-block (32 values of a Q4_K block, 16 of a
+// Q6_K block), its values and codes in registers, every loop over them unrolled.
+// The fits are sequential f32 sums that have to keep their order, so a lane is
+// the smallest unit; the lanes of a block then agree on the block's scales with
+// DPP exchanges and write its bytes 16 at a time.
+//
+// What bounds them: VALU issue (Q4_K: five passes of ~12 instructions a value).
+// A wave stages its 64 sub-blocks through LDS, because a lane's own values are
+// contiguous and reading them directly would touch 64 lines per load.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int round_i(float v) {
   // f32::round (ties away from zero) then a saturating cast to i32.
@@ -129,43 +145,55 @@ __device__ __forceinline__ int round_i(float v) {
   return (int)r;
 }
 
-__device__ __forceinline__ int clamp_i(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
+// round(v) clamped to [0, hi] as an integer-valued float: f32::round (ties away
+// from zero) and a saturating cast, of which NaN gives 0. For v >= 0 that is
+// floor(v + 0.5 - 2^-25): the sum rounds up to the next integer exactly from
+// .5 on (with 0.5 itself 0.5 - 2^-25 would round to 1).
+__device__ __forceinline__ float round_to(float v, float hi) {
+  return fminf(floorf(fmaxf(v, 0.0f) + 0.49999997f), hi);
+}
 
-// Asymmetric fit of n values to [0, nmax] codes (make_qkx1_quants); returns
-// the scale and writes the (positive) offset `-min`.
-__device__ float fit_qkx1(int nmax, int ntry, const float* x, int n, float* neg_min) {
+// The same for a signed range.
+__device__ __forceinline__ float round_between(float v, float lo, float hi) {
+  const float r = fminf(fmaxf(truncf(v + copysignf(0.49999997f, v)), lo), hi);
+  return v == v ? r : 0.0f;
+}
+
+// Asymmetric fit of 32 values to [0, 15] codes, five tries (make_qkx1_quants);
+// returns the scale and the (positive) offset `-min`.
+__device__ __forceinline__ float fit_q4(const float (&x)[32], float* neg_min) {
 #pragma clang fp contract(off)
-  uint8_t codes[32];
-  for (int i = 0; i < n; ++i) codes[i] = 0;
+  float c[32];
   float lo = x[0], hi = x[0];
-  for (int i = 1; i < n; ++i) {
+#pragma unroll
+  for (int i = 1; i < 32; ++i) {
     if (x[i] < lo) lo = x[i];
     if (x[i] > hi) hi = x[i];
   }
-  if (hi == lo) {
-    *neg_min = 0.0f;
-    return 0.0f;
-  }
+#pragma unroll
+  for (int i = 0; i < 32; ++i) c[i] = 0.0f;
+  *neg_min = 0.0f;
+  if (hi == lo) return 0.0f;
   float mn = fminf(lo, 0.0f);
-  float iscale = (float)nmax / (hi - mn);
+  float iscale = 15.0f / (hi - mn);
   float scale = 1.0f / iscale;
-  for (int it = 0; it < ntry; ++it) {
-    float sumlx = 0.0f;
-    int suml2 = 0;
+#pragma unroll 1
+  for (int it = 0; it < 5; ++it) {
+    float sumlx = 0.0f, suml2 = 0.0f;  // suml2 counts exactly: at most 32 * 225
     bool changed = false;
-    for (int i = 0; i < n; ++i) {
-      const int c = clamp_i(round_i(iscale * (x[i] - mn)), 0, nmax);
-      if ((uint8_t)c != codes[i]) {
-        codes[i] = (uint8_t)c;
-        changed = true;
-      }
-      sumlx += (x[i] - mn) * (float)c;
-      suml2 += c * c;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const float d = x[i] - mn, n = round_to(iscale * d, 15.0f);
+      changed |= n != c[i];
+      c[i] = n;
+      sumlx += d * n;
+      suml2 += n * n;
     }
-    scale = sumlx / (float)suml2;
+    scale = sumlx / suml2;
     float acc = 0.0f;
-    for (int i = 0; i < n; ++i) acc += x[i] - scale * (float)codes[i];
-    mn = acc / (float)n;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc += x[i] - scale * c[i];
+    mn = acc / 32.0f;
     if (mn > 0.0f) mn = 0.0f;
     iscale = 1.0f / scale;
     if (!changed) break;
@@ -184,176 +212,239 @@ __device__ __forceinline__ void q4k_scale_min(int j, const uint8_t* s, int* sc, 
   }
 }
 
-__device__ void q4k_quantize_block(const float* __restrict__ x, uint8_t* __restrict__ out) {
-#pragma clang fp contract(off)
-  float sub_scale[8], sub_min[8];
-  for (int j = 0; j < 8; ++j) sub_scale[j] = fit_qkx1(15, 5, x + 32 * j, 32, &sub_min[j]);
-  float max_scale = 0.0f, max_min = 0.0f;
-  for (int j = 0; j < 8; ++j) max_scale = fmaxf(sub_scale[j], max_scale);
-  for (int j = 0; j < 8; ++j) max_min = fmaxf(sub_min[j], max_min);
-  const float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
-  const float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
-  uint8_t sc[12];
-  for (int i = 0; i < 12; ++i) sc[i] = 0;
-  for (int j = 0; j < 8; ++j) {
-    int ls = round_i(inv_scale * sub_scale[j]);
-    int lm = round_i(inv_min * sub_min[j]);
-    ls = ls < 63 ? ls : 63;
-    lm = lm < 63 ? lm : 63;
-    if (j < 4) {
-      sc[j] = (uint8_t)ls;
-      sc[j + 4] = (uint8_t)lm;
-    } else {
-      sc[j + 4] = (uint8_t)((ls & 0x0f) | ((lm & 0x0f) << 4));
-      sc[j - 4] |= (uint8_t)((ls >> 4) << 6);
-      sc[j] |= (uint8_t)((lm >> 4) << 6);
-    }
-  }
-  const uint16_t dh = f2h(max_scale / 63.0f);
-  const uint16_t mh = f2h(max_min / 63.0f);
-  const float df = h2f(dh), mf = h2f(mh);
-  uint8_t codes[256];
-  for (int i = 0; i < 256; ++i) codes[i] = 0;
-  for (int j = 0; j < 8; ++j) {
-    int s, m;
-    q4k_scale_min(j, sc, &s, &m);
-    const float d = df * (float)s;
-    if (d == 0.0f) continue;
-    const float dm = mf * (float)m;
-    for (int i = 0; i < 32; ++i) codes[32 * j + i] = (uint8_t)clamp_i(round_i((x[32 * j + i] + dm) / d), 0, 15);
-  }
-  out[0] = (uint8_t)dh;
-  out[1] = (uint8_t)(dh >> 8);
-  out[2] = (uint8_t)mh;
-  out[3] = (uint8_t)(mh >> 8);
-  for (int i = 0; i < 12; ++i) out[4 + i] = sc[i];
-  for (int c = 0; c < 4; ++c)
-    for (int i = 0; i < 32; ++i)
-      out[16 + 32 * c + i] = (uint8_t)(codes[64 * c + i] | (codes[64 * c + 32 + i] << 4));
+// v of the lane whose index differs in the low bits of MASK (1, 2 or 4)
+template <int MASK>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  static_assert(MASK == 1 || MASK == 2 || MASK == 4, "");
+  if constexpr (MASK == 4) return (uint32_t)__shfl_xor((int)v, 4);
+  return (uint32_t)dpp_i<MASK == 1 ? 0xb1 : 0x4e>((int)v);
+}
+__device__ __forceinline__ float fmax8(float v) {  // over the 8 lanes of a block, from 0
+  v = fmaxf(fmaxf(v, 0.0f), dpp_f<0xb1>(v));
+  v = fmaxf(v, dpp_f<0x4e>(v));
+  return fmaxf(v, dpp_f<0x141>(v));
 }
 
-// ---------------------------------------------------------------------------
-// Q6_K weight quantizer (one thread per super-block).
-// ---------------------------------------------------------------------------
+// The wave's 64 sub-blocks of N values: `first` is the first one's index, `total`
+// their number. Coalesced 16-byte loads into LDS (chunk c of sub-block r in slot
+// c ^ r % (N / 4)), then each lane's own values. Lanes past the end repeat the
+// last sub-block.
+template <int N>
+__device__ __forceinline__ void load_sub_block(const float* __restrict__ w, long long first, long long total,
+                                               float* lds, int lane, float (&x)[N]) {
+  constexpr int C = N / 4;
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  f32x4* l4 = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int s = 64 * i + lane, r = s / C, c = s % C;
+    const float* p = w + (first + r < total ? first + r : total - 1) * N + 4 * c;
+    l4[r * C + (c ^ (r % C))] = (f32x4){p[0], p[1], p[2], p[3]};
+  }
+  // (a wave reads only what it wrote itself: LDS keeps a wave's order)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const f32x4 v = l4[lane * C + (c ^ (lane % C))];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[4 * c + e] = v[e];
+  }
+}
 
-// Symmetric fit of 16 values to [-nmax, nmax-1] with the squared-value
-// weighting (make_qx_quants with rmse_type 1); codes are stored biased by nmax.
-__device__ float fit_qx16(int nmax, const float* x, int8_t* codes) {
+// Q4_K blocks: 8 lanes each.
+__device__ __forceinline__ void quantize_q4k_lanes(const float* __restrict__ w, uint8_t* __restrict__ out,
+                                                   long long nblocks, float* lds) {
 #pragma clang fp contract(off)
-  const int n = 16;
+  const int lane = threadIdx.x & 63, j = lane & 7;
+  const long long first = ((long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64;
+  if (first >= 8 * nblocks) return;
+  float x[32];
+  load_sub_block<32>(w, first, 8 * nblocks, lds, lane, x);
+  float sub_min;
+  const float sub_scale = fit_q4(x, &sub_min);
+  const float max_scale = fmax8(sub_scale), max_min = fmax8(sub_min);
+  const float inv_scale = max_scale > 0.0f ? 63.0f / max_scale : 0.0f;
+  const float inv_min = max_min > 0.0f ? 63.0f / max_min : 0.0f;
+  int ls = round_i(inv_scale * sub_scale);
+  int lm = round_i(inv_min * sub_min);
+  ls = ls < 63 ? ls : 63;
+  lm = lm < 63 ? lm : 63;
+  // the scale bytes: lanes 0-3 hold bytes j and j + 4 (own low bits, lane j + 4's
+  // top two), lanes 4-7 byte j + 4 (own low nibbles)
+  const int pls = (int)lane_xor<4>((uint32_t)ls), plm = (int)lane_xor<4>((uint32_t)lm);
+  const uint32_t a = (uint32_t)((ls & 0xff) | (((pls >> 4) << 6) & 0xff));
+  const uint32_t b = (uint32_t)((lm & 0xff) | (((plm >> 4) << 6) & 0xff));
+  const uint32_t c = (uint32_t)((ls & 0x0f) | ((lm & 0x0f) << 4));
+  const uint32_t pa = lane_xor<4>(a), pb = lane_xor<4>(b);
+  const int s = j < 4 ? (int)(a & 63) : (int)((c & 0x0f) | ((pa >> 6) << 4));
+  const int m = j < 4 ? (int)(b & 63) : (int)((c >> 4) | ((pb >> 6) << 4));
+  const uint16_t dh = f2h(max_scale / 63.0f), mh = f2h(max_min / 63.0f);
+  const float d = h2f(dh) * (float)s, dm = h2f(mh) * (float)m;
+  uint32_t q[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    q[i] = 0;
+    if (d != 0.0f) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) q[i] |= (uint32_t)round_to((x[4 * i + e] + dm) / d, 15.0f) << (8 * e);
+    }
+  }
+  // quad-wide OR: dword of bytes 0-3 / 4-7 in lanes 0-3, of bytes 8-11 in lanes 4-7
+  auto gather = [&](uint32_t v) {
+    v <<= 8 * (j & 3);
+    v |= lane_xor<1>(v);
+    return v | lane_xor<2>(v);
+  };
+  const uint32_t ga = gather(a), gb = gather(b), gc = lane_xor<4>(gather(c));
+  // lanes 2i, 2i + 1 share 32 bytes of quants (low and high nibbles): each writes 16
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t give = (j & 1) ? q[i] : q[4 + i], keep = (j & 1) ? q[4 + i] : q[i];
+    const uint32_t got = lane_xor<1>(give);
+    o[i] = (j & 1) ? got | keep << 4 : keep | got << 4;
+  }
+  if (first + lane >= 8 * nblocks) return;
+  uint4* blk = reinterpret_cast<uint4*>(out + kQ4KBytes * ((first + lane) >> 3));
+  if (j == 0) blk[0] = make_uint4((uint32_t)dh | (uint32_t)mh << 16, ga, gb, gc);
+  blk[1 + j] = make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// Symmetric fit of 16 values to [-32, 31] with the squared-value weighting
+// (make_qx_quants with rmse_type 1); codes are integer-valued floats.
+__device__ __forceinline__ float fit_q6(const float (&x)[16], float (&codes)[16]) {
+#pragma clang fp contract(off)
   float amax = 0.0f, vmax = 0.0f;
-  for (int i = 0; i < n; ++i) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
     const float a = fabsf(x[i]);
     if (a > amax) {
       amax = a;
       vmax = x[i];
     }
   }
-  if (amax == 0.0f) {
-    for (int i = 0; i < n; ++i) codes[i] = 0;
-    return 0.0f;
-  }
-  float iscale = -(float)nmax / vmax;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) codes[i] = -32.0f;  // stored as 0 where every value is 0
+  if (amax == 0.0f) return 0.0f;
+  const float iscale = -32.0f / vmax;
   float sumlx = 0.0f, suml2 = 0.0f;
-  for (int i = 0; i < n; ++i) {
-    const int l = clamp_i(round_i(iscale * x[i]), -nmax, nmax - 1);
-    codes[i] = (int8_t)(l + nmax);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float l = round_between(iscale * x[i], -32.0f, 31.0f);
+    codes[i] = l;
     const float w = x[i] * x[i];
-    const float lf = (float)l;
-    sumlx += w * x[i] * lf;
-    suml2 += w * lf * lf;
+    sumlx += w * x[i] * l;
+    suml2 += w * l * l;
   }
   float scale = sumlx / suml2;
   float best = scale * sumlx;
+#pragma unroll 1
   for (int t = 0; t < 3; ++t) {
     const float is = 1.0f / scale;
-    float slx = 0.0f, sl2 = 0.0f;
+    float slx = 0.0f, sl2 = 0.0f, n[16];
     bool changed = false;
-    for (int i = 0; i < n; ++i) {
-      const int l = clamp_i(round_i(is * x[i]), -nmax, nmax - 1);
-      if (l + nmax != codes[i]) changed = true;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      n[i] = round_between(is * x[i], -32.0f, 31.0f);
+      changed |= n[i] != codes[i];
       const float w = x[i] * x[i];
-      const float lf = (float)l;
-      slx += w * x[i] * lf;
-      sl2 += w * lf * lf;
+      slx += w * x[i] * n[i];
+      sl2 += w * n[i] * n[i];
     }
     if (!changed || sl2 == 0.0f || slx * slx <= best * sl2) break;
-    for (int i = 0; i < n; ++i) codes[i] = (int8_t)(nmax + clamp_i(round_i(is * x[i]), -nmax, nmax - 1));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) codes[i] = n[i];
     sumlx = slx;
     suml2 = sl2;
     scale = sumlx / suml2;
     best = scale * sumlx;
   }
+#pragma unroll 1
   for (int t = 0; t < 5; ++t) {
-    int n_changed = 0;
-    for (int i = 0; i < n; ++i) {
-      const float w = x[i] * x[i];
-      const int l = codes[i] - nmax;
-      float slx = sumlx - w * x[i] * (float)l;
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float w = x[i] * x[i], l = codes[i];
+      float slx = sumlx - w * x[i] * l;
       if (slx > 0.0f) {
-        float sl2 = suml2 - w * (float)l * (float)l;
-        const int nl = clamp_i(round_i(x[i] * sl2 / slx), -nmax, nmax - 1);
+        float sl2 = suml2 - w * l * l;
+        const float nl = round_between(x[i] * sl2 / slx, -32.0f, 31.0f);
         if (nl != l) {
-          slx += w * x[i] * (float)nl;
-          sl2 += w * (float)nl * (float)nl;
+          slx += w * x[i] * nl;
+          sl2 += w * nl * nl;
           if (sl2 > 0.0f && slx * slx * suml2 > sumlx * sumlx * sl2) {
-            codes[i] = (int8_t)(nmax + nl);
+            codes[i] = nl;
             sumlx = slx;
             suml2 = sl2;
             scale = sumlx / suml2;
-            best = scale * sumlx;
-            ++n_changed;
+            any = true;
           }
         }
       }
     }
-    if (n_changed == 0) break;
+    if (!any) break;
   }
   return scale;
 }
 
-__device__ void q6k_quantize_block(const float* __restrict__ x, uint8_t* __restrict__ out) {
+// Q6_K blocks in the device layout (bodies, then the f16 scales): 16 lanes each.
+__device__ __forceinline__ void quantize_q6k_lanes(const float* __restrict__ w, uint8_t* __restrict__ out,
+                                                   long long nblocks, float* lds) {
 #pragma clang fp contract(off)
-  int8_t codes[256];
-  float scales[16];
-  float max_scale = 0.0f, max_abs = 0.0f;
-  for (int ib = 0; ib < 16; ++ib) {
-    const float s = fit_qx16(32, x + 16 * ib, codes + 16 * ib);
-    scales[ib] = s;
-    const float a = fabsf(s);
-    if (a > max_abs) {
-      max_abs = a;
-      max_scale = s;
-    }
-  }
+  const int lane = threadIdx.x & 63, j = lane & 15;
+  const long long first = ((long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 64;
+  if (first >= 16 * nblocks) return;
+  float x[16], codes[16];
+  load_sub_block<16>(w, first, 16 * nblocks, lds, lane, x);
+  const float scale = fit_q6(x, codes);
+  // the first sub-block scale of the largest magnitude (0 if none is above 0)
+  const float a = fabsf(scale) > 0.0f ? fabsf(scale) : 0.0f;
+  float amax = fmaxf(a, dpp_f<0xb1>(a));
+  amax = fmaxf(amax, dpp_f<0x4e>(amax));
+  amax = fmaxf(amax, dpp_f<0x141>(amax));
+  amax = fmaxf(amax, dpp_f<0x140>(amax));
+  int at = a == amax && amax > 0.0f ? j : 16;
+  at = min(at, dpp_i<0xb1>(at));
+  at = min(at, dpp_i<0x4e>(at));
+  at = min(at, dpp_i<0x141>(at));
+  at = min(at, dpp_i<0x140>(at));
+  const float first_max = __shfl(scale, (lane & 48) + (at & 15));
+  const float max_scale = at < 16 ? first_max : 0.0f;
   const float iscale = -128.0f / max_scale;
   const uint16_t dh = f2h(1.0f / iscale);
-  int8_t sc8[16];
-  for (int j = 0; j < 16; ++j) {
-    const int v = round_i(iscale * scales[j]);
-    sc8[j] = (int8_t)(v < 127 ? v : 127);
+  const int v = round_i(iscale * scale);
+  const int8_t sc = (int8_t)(v < 127 ? v : 127);
+  const float d = h2f(dh) * (float)sc;
+  if (!(d == 0.0f)) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) codes[i] = round_between(x[i] / d, -32.0f, 31.0f);
   }
-  const float df = h2f(dh);
-  for (int j = 0; j < 16; ++j) {
-    const float d = df * (float)sc8[j];
-    if (d == 0.0f) continue;
-    for (int i = 0; i < 16; ++i)
-      codes[16 * j + i] = (int8_t)(clamp_i(round_i(x[16 * j + i] / d), -32, 31) + 32);
-  }
-  uint8_t* ql = out;
-  uint8_t* qh = out + 128;
-  for (int h = 0; h < 2; ++h) {
-    const int8_t* c = codes + 128 * h;
-    for (int l = 0; l < 32; ++l) {
-      ql[64 * h + l] = (uint8_t)((c[l] & 0xf) | ((c[l + 64] & 0xf) << 4));
-      ql[64 * h + 32 + l] = (uint8_t)((c[l + 32] & 0xf) | ((c[l + 96] & 0xf) << 4));
-      qh[32 * h + l] = (uint8_t)(((c[l] >> 4) & 3) | (((c[l + 32] >> 4) & 3) << 2) |
-                                 (((c[l + 64] >> 4) & 3) << 4) | (((c[l + 96] >> 4) & 3) << 6));
+  // lane j = 8 h + 2 g + p: values 128 h + 32 g + 16 p ...; quants of g and g + 2
+  // share bytes (low and high nibbles), the top two bits of the four g share one
+  const int h = j >> 3, g = (j >> 1) & 3, p = j & 1;
+  uint32_t lo[4], hi[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    lo[i] = hi[i] = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t c = (uint32_t)((int)codes[4 * i + e] + 32);
+      lo[i] |= (c & 15) << (8 * e);
+      hi[i] |= ((c >> 4) & 3) << (8 * e + 2 * g);
     }
+    lo[i] |= lane_xor<4>(lo[i]) << 4;  // of use in lanes g < 2
+    hi[i] |= lane_xor<2>(hi[i]);
+    hi[i] |= lane_xor<4>(hi[i]);
   }
-  for (int j = 0; j < 16; ++j) out[192 + j] = (uint8_t)sc8[j];
-  out[208] = (uint8_t)dh;
-  out[209] = (uint8_t)(dh >> 8);
+  const long long blk = (first + lane) >> 4;
+  if (blk >= nblocks) return;
+  uint8_t* body = out + kQ6KBody * blk;
+  if (g < 2) *reinterpret_cast<uint4*>(body + 64 * h + 32 * g + 16 * p) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+  if (g == 2) *reinterpret_cast<uint4*>(body + 128 + 32 * h + 16 * p) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+  body[192 + j] = (uint8_t)sc;
+  if (j == 0) reinterpret_cast<uint16_t*>(out + kQ6KBody * nblocks)[blk] = dh;
 }
 
 }  // namespace qmm
@@ -386,21 +477,37 @@ extern "C" __global__ void __launch_bounds__(256) qmm_quantize_q8_0(const float*
   qmm::q80_block(x + row * ldx + 32LL * b, y + bc * qmm::kQ80Bytes, (int)(t & 7), valid);
 }
 
-// Weight quantizers to GGML bytes: one thread per super-block.
-extern "C" __global__ void __launch_bounds__(64) qmm_quantize_q4k_w(const float* __restrict__ w,
-                                                                   uint8_t* __restrict__ out,
-                                                                   long long nblocks) {
-  const long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nblocks) return;
-  qmm::q4k_quantize_block(w + 256 * b, out + qmm::kQ4KBytes * b);
+// Weight quantizers to the device layout, four waves of 64 sub-blocks. One
+// qmm_qtensor_quantize call on 4096 x 4096 values (allocation and a
+// synchronisation included): Q4_K 65 us, Q6_K 103 us; with one thread per
+// super-block and its codes in byte arrays (scratch memory) 983 us and 402 us.
+extern "C" __global__ void __launch_bounds__(256) qmm_quantize_q4k_w(const float* __restrict__ w,
+                                                                     uint8_t* __restrict__ out, long long nblocks) {
+  __shared__ __attribute__((aligned(16))) float lds[4][64 * 32];
+  qmm::quantize_q4k_lanes(w, out, nblocks, lds[threadIdx.x >> 6]);
 }
 
-extern "C" __global__ void __launch_bounds__(64) qmm_quantize_q6k_w(const float* __restrict__ w,
-                                                                   uint8_t* __restrict__ out,
-                                                                   long long nblocks) {
-  const long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= nblocks) return;
-  qmm::q6k_quantize_block(w + 256 * b, out + qmm::kQ6KBytes * b);
+extern "C" __global__ void __launch_bounds__(256) qmm_quantize_q6k_w(const float* __restrict__ w,
+                                                                     uint8_t* __restrict__ out, long long nblocks) {
+  __shared__ __attribute__((aligned(16))) float lds[4][64 * 16];
+  qmm::quantize_q6k_lanes(w, out, nblocks, lds[threadIdx.x >> 6]);
+}
+
+// Q8_0 weights straight to the device layout (quants, then the f16 scales): the
+// call takes 40 us on 4096 x 4096 values, 82 us by way of GGML blocks in a
+// buffer of their own.
+extern "C" __global__ void __launch_bounds__(256) qmm_quantize_q8_0_w(const float* __restrict__ w,
+                                                                      uint8_t* __restrict__ out, long long nblocks) {
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long blk = t >> 3;
+  const bool valid = blk < nblocks;
+  const float* x = w + (valid ? 4 * t : 0);
+  const float e[4] = {x[0], x[1], x[2], x[3]};
+  uint16_t d;
+  const uint32_t q = qmm::q80_lane(e, &d);
+  if (!valid) return;
+  reinterpret_cast<uint32_t*>(out)[t] = q;
+  if ((t & 7) == 0) reinterpret_cast<uint16_t*>(out + qmm::kQ80Body * nblocks)[blk] = d;
 }
 
 // GGML bytes <-> device layout for the formats whose blocks are not 16-byte
