@@ -437,8 +437,9 @@ int qmm_qtensor_dequantize_to(const qmm_qtensor* t, void* dst, int out_dtype, vo
   void* a1 = dst;
   int f = fmt;
   void* args[] = {&a0, &a1, &nblocks, &f};
-  const long long threads = fmt == kFmtQ80 ? nblocks : nblocks * 8;
-  return launch(d, name, ceil_div(threads, 256), 256, 0, (hipStream_t)stream, args);
+  // a thread forms 16 bytes of outputs in each of kDqUnits (4) units
+  const long long units = t->n * t->k * (out_dtype == QMM_F32 ? 4 : 2) / 16;
+  return launch(d, name, ceil_div(units, 4 * 256), 256, 0, (hipStream_t)stream, args);
 }
 
 int qmm_qtensor_dequantize(const qmm_qtensor* t, float* dst, void* stream) {

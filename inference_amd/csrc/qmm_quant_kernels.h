@@ -547,70 +547,176 @@ extern "C" __global__ void qmm_dev_to_ggml(const uint8_t* __restrict__ src, uint
   }
 }
 
-// Dequantize a device-layout tensor (QTensor::dequantize). One thread per 32
-// consecutive outputs; formulas of crates/llm/mlx-llm/src/gguf/dequant.rs
-// :284-290 (Q8_0), :391-416 (Q4_K), :452-474 (Q6_K), one rounding per f32
-// operation; the f16 / bf16 outputs round the f32 value once more, to
-// nearest even (the f32 dequantize followed by to_dtype).
+// Dequantize a device-layout tensor (QTensor::dequantize); formulas of
+// crates/llm/mlx-llm/src/gguf/dequant.rs:284-290 (Q8_0), :391-416 (Q4_K),
+// :452-474 (Q6_K), one rounding per f32 operation; the f16 / bf16 outputs round
+// the f32 value once more, to nearest even (the f32 dequantize followed by
+// to_dtype; a NaN stays one).
+//
+// Bound by memory: a thread forms 16 bytes of consecutive outputs (4 f32 or 8
+// 16-bit values, always inside one sub-block), so that a wave's loads and stores
+// are whole lines, and kDqUnits of them 256 threads apart, so that their loads
+// are in flight together. 14336 x 4096 Q8_0 to f32 (295 MB) took 93 us with one
+// thread per 32 consecutive values, 128 bytes from its neighbour's, and its
+// conversion to bf16 63 us; to bf16 at once (180 MB) it takes 29 us.
 namespace qmm {
-__device__ __forceinline__ void put_val(float* y, long long i, float v) { y[i] = v; }
-__device__ __forceinline__ void put_val(_Float16* y, long long i, float v) { y[i] = (_Float16)v; }
-__device__ __forceinline__ void put_val(uint16_t* y, long long i, float v) {  // bf16, round to nearest even
+constexpr int kDqUnits = 4;
+
+__device__ __forceinline__ uint32_t bf16_bits(float v) {  // round to nearest even
   const uint32_t b = __builtin_bit_cast(uint32_t, v);
-  y[i] = (uint16_t)((b + 0x7fffu + ((b >> 16) & 1u)) >> 16);
+  return v == v ? (b + 0x7fffu + ((b >> 16) & 1u)) >> 16 : 0x7fc0u;
+}
+__device__ __forceinline__ void put_vals(float* y, const float (&v)[4]) {
+  *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void put_vals(_Float16* y, const float (&v)[8]) {
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = v[2 * i], b = v[2 * i + 1];
+    // the f32 product first: folded into its conversion as v_fma_mixlo_f16 x, y, 0
+    // a -0 would come out as +0
+    asm("" : "+v"(a), "+v"(b));
+    w[i] = (uint32_t)f2h(a) | (uint32_t)f2h(b) << 16;
+  }
+  *reinterpret_cast<uint4*>(y) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+__device__ __forceinline__ void put_vals(uint16_t* y, const float (&v)[8]) {  // bf16
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = bf16_bits(v[2 * i]) | bf16_bits(v[2 * i + 1]) << 16;
+  *reinterpret_cast<uint4*>(y) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+__device__ __forceinline__ void put_val(float* y, float v) { *y = v; }
+__device__ __forceinline__ void put_val(_Float16* y, float v) {
+  asm("" : "+v"(v));
+  *y = (_Float16)v;
+}
+__device__ __forceinline__ void put_val(uint16_t* y, float v) { *y = (uint16_t)bf16_bits(v); }
+
+// N consecutive bytes (4 or 8, aligned) as dwords
+template <int N>
+struct Bytes {
+  uint32_t w[N / 4];
+  __device__ __forceinline__ uint32_t operator[](int i) const { return (w[i / 4] >> (8 * (i % 4))) & 0xffu; }
+};
+template <int N>
+__device__ __forceinline__ Bytes<N> load_bytes(const uint8_t* p) {
+  Bytes<N> b;
+  if constexpr (N == 4) {
+    b.w[0] = *reinterpret_cast<const uint32_t*>(p);
+  } else {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    b.w[0] = v.x;
+    b.w[1] = v.y;
+  }
+  return b;
+}
+
+// What a unit (outputs N u .. N u + N - 1) needs from memory, and its values.
+template <int FMT, int N>
+struct DqUnit {
+  Bytes<N> q, h;     // quants; Q6_K: their top bits
+  uint4 head;        // Q4_K: d, dmin and the scale bytes
+  uint16_t d;        // Q6_K, Q8_0
+  int8_t sc;         // Q6_K
+  __device__ __forceinline__ void load(const uint8_t* __restrict__ src, long long u, long long nblocks) {
+    if constexpr (FMT == kFmtQ80) {
+      q = load_bytes<N>(src + N * u);
+      d = reinterpret_cast<const uint16_t*>(src + kQ80Body * nblocks)[u / (32 / N)];
+    } else {
+      const long long b = u / (256 / N);
+      const int e = (int)(u % (256 / N)) * N, part = e / 32, l = e % 32;
+      if constexpr (FMT == kFmtQ4K) {
+        const uint8_t* blk = src + kQ4KBytes * b;
+        head = *reinterpret_cast<const uint4*>(blk);
+        q = load_bytes<N>(blk + 16 + 32 * (part >> 1) + l);
+      } else {
+        // outputs 128 h + 32 s + [0, 32): low / high nibbles of ql, 2 bits of qh
+        const uint8_t* body = src + kQ6KBody * b;
+        const int hf = part >> 2, s = part & 3;
+        q = load_bytes<N>(body + 64 * hf + 32 * (s & 1) + l);
+        h = load_bytes<N>(body + 128 + 32 * hf + l);
+        sc = (int8_t)body[192 + 8 * hf + 2 * s + l / 16];
+        d = reinterpret_cast<const uint16_t*>(src + kQ6KBody * nblocks)[b];
+      }
+    }
+  }
+  __device__ __forceinline__ void values(long long u, float (&v)[N]) const {
+#pragma clang fp contract(off)
+    if constexpr (FMT == kFmtQ80) {
+      const float df = h2f(d);
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = (float)(int8_t)q[i] * df;
+      return;
+    }
+    const int part = (int)(u % (256 / N)) * N / 32;
+    if constexpr (FMT == kFmtQ4K) {
+      const uint32_t hw[4] = {head.x, head.y, head.z, head.w};
+      // q4k_scale_min on the header's dwords: bytes 0-3, 4-7 and 8-11 are hw[1..3]
+      const int j = part & 3, o = 8 * j;
+      const uint32_t a = (hw[1] >> o) & 0xff, b = (hw[2] >> o) & 0xff, c = (hw[3] >> o) & 0xff;
+      const uint32_t sc4 = part < 4 ? a & 63 : (c & 0x0f) | (a >> 6) << 4;
+      const uint32_t mn4 = part < 4 ? b & 63 : (c >> 4) | (b >> 6) << 4;
+      const float d1 = h2f(hw[0]) * (float)(int)sc4, m1 = h2f(hw[0] >> 16) * (float)(int)mn4;
+      const int sh = (part & 1) * 4;
+#pragma unroll
+      for (int i = 0; i < N; ++i) v[i] = d1 * (float)(int)((q[i] >> sh) & 0xf) - m1;
+    } else {
+      const int s = part & 3, nsh = (s >> 1) * 4, hsh = 2 * s;
+      const float ds = h2f(d) * (float)sc;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        v[i] = ds * (float)((int)(((q[i] >> nsh) & 0xf) | (((h[i] >> hsh) & 3) << 4)) - 32);
+    }
+  }
+};
+
+template <int FMT, class T>
+__device__ __forceinline__ void dequantize_units(const uint8_t* __restrict__ src, T* __restrict__ y, long long nblocks) {
+  constexpr int N = 16 / (int)sizeof(T);
+  const long long units = nblocks * ((FMT == kFmtQ80 ? 32 : 256) / N);
+  const long long u0 = (long long)blockIdx.x * (256 * kDqUnits) + threadIdx.x;
+  const bool aligned = (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+  DqUnit<FMT, N> unit[kDqUnits];
+#pragma unroll
+  for (int i = 0; i < kDqUnits; ++i) unit[i].load(src, min(u0 + 256 * i, units - 1), nblocks);
+#pragma unroll
+  for (int i = 0; i < kDqUnits; ++i) {
+    const long long u = u0 + 256 * i;
+    if (u >= units) return;
+    float v[N];
+    unit[i].values(u, v);
+    if (aligned) {
+      put_vals(y + N * u, v);
+    } else {  // a destination off the 16-byte grid: value by value
+#pragma unroll
+      for (int j = 0; j < N; ++j) put_val(y + N * u + j, v[j]);
+    }
+  }
 }
 
 template <class T>
 __device__ __forceinline__ void dequantize_blocks(const uint8_t* __restrict__ src, T* __restrict__ y,
                                                   long long nblocks, int fmt) {
-#pragma clang fp contract(off)
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (fmt == kFmtQ80) {
-    if (t >= nblocks) return;
-    const int8_t* q = reinterpret_cast<const int8_t*>(src + kQ80Body * t);
-    const float d = h2f(reinterpret_cast<const uint16_t*>(src + kQ80Body * nblocks)[t]);
-    for (int j = 0; j < 32; ++j) put_val(y, 32 * t + j, (float)q[j] * d);
-    return;
-  }
-  const long long b = t >> 3;
-  const int part = (int)(t & 7);
-  if (b >= nblocks) return;
-  const long long o = 256 * b + 32 * part;
-  if (fmt == kFmtQ4K) {
-    const uint8_t* blk = src + kQ4KBytes * b;
-    const float d = h2f(blk[0] | (blk[1] << 8)), dmin = h2f(blk[2] | (blk[3] << 8));
-    int sc, m;
-    q4k_scale_min(part, blk + 4, &sc, &m);
-    const float d1 = d * (float)sc, m1 = dmin * (float)m;
-    const uint8_t* qs = blk + 16 + 32 * (part >> 1);
-    const int sh = (part & 1) * 4;
-    for (int l = 0; l < 32; ++l) put_val(y, o + l, d1 * (float)((qs[l] >> sh) & 0xf) - m1);
-  } else {
-    const uint8_t* body = src + kQ6KBody * b;
-    const float d = h2f(reinterpret_cast<const uint16_t*>(src + kQ6KBody * nblocks)[b]);
-    const int8_t* sc = reinterpret_cast<const int8_t*>(body + 192);
-    // outputs 128h + 32s + [0, 32): ql low/high nibble and 2 bits of qh.
-    const int h = part >> 2, s = part & 3;
-    const uint8_t* ql = body + 64 * h + 32 * (s & 1);
-    const uint8_t* qh = body + 128 + 32 * h;
-    const int nsh = (s >> 1) * 4, hsh = 2 * s;
-    for (int l = 0; l < 32; ++l) {
-      const int q = (((ql[l] >> nsh) & 0xf) | (((qh[l] >> hsh) & 3) << 4)) - 32;
-      put_val(y, o + l, d * (float)sc[8 * h + 2 * s + l / 16] * (float)q);
-    }
-  }
+  if (fmt == kFmtQ80) return dequantize_units<kFmtQ80>(src, y, nblocks);
+  if (fmt == kFmtQ4K) return dequantize_units<kFmtQ4K>(src, y, nblocks);
+  dequantize_units<kFmtQ6K>(src, y, nblocks);
 }
 }  // namespace qmm
 
-extern "C" __global__ void qmm_dequantize(const uint8_t* __restrict__ src, float* __restrict__ y, long long nblocks,
-                                          int fmt) {
+extern "C" __global__ void __launch_bounds__(256) qmm_dequantize(const uint8_t* __restrict__ src,
+                                                                 float* __restrict__ y, long long nblocks, int fmt) {
   qmm::dequantize_blocks(src, y, nblocks, fmt);
 }
-extern "C" __global__ void qmm_dequantize_f16(const uint8_t* __restrict__ src, _Float16* __restrict__ y,
-                                              long long nblocks, int fmt) {
+extern "C" __global__ void __launch_bounds__(256) qmm_dequantize_f16(const uint8_t* __restrict__ src,
+                                                                     _Float16* __restrict__ y, long long nblocks,
+                                                                     int fmt) {
   qmm::dequantize_blocks(src, y, nblocks, fmt);
 }
-extern "C" __global__ void qmm_dequantize_bf16(const uint8_t* __restrict__ src, uint16_t* __restrict__ y,
-                                               long long nblocks, int fmt) {
+extern "C" __global__ void __launch_bounds__(256) qmm_dequantize_bf16(const uint8_t* __restrict__ src,
+                                                                      uint16_t* __restrict__ y, long long nblocks,
+                                                                      int fmt) {
   qmm::dequantize_blocks(src, y, nblocks, fmt);
 }

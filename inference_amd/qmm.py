@@ -427,7 +427,9 @@ class QLinear:
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.strategy == MatmulStrategy.DEQUANT_DENSE:
-            w = self.weight.dequantize(torch.float32).to(x.dtype)
+            # f16 / bf16 weights are the f32 values rounded once: formed directly, without the f32 copy
+            direct = x.dtype in (torch.float32, torch.float16, torch.bfloat16)
+            w = self.weight.dequantize(x.dtype if direct else torch.float32).to(x.dtype)
             b = self.bias.to(x.dtype) if self.bias is not None else None
             return torch.nn.functional.linear(x, w, b)
         y = self._mm.forward(x.to(torch.float32).contiguous())

@@ -116,3 +116,26 @@ def test_quantize_onto_equals_device_quantize():
         a = QTensor.quantize_onto(w, dt, DEV)
         b = QTensor.quantize(w.to(DEV), dt)
         assert a.device == DEV and np.array_equal(a.to_ggml(), b.to_ggml())
+
+
+@pytest.mark.parametrize("dt", [GgmlDType.Q8_0, GgmlDType.Q4K, GgmlDType.Q6K])
+@pytest.mark.parametrize("n,k", [(1, 256), (5, 256), (33, 768)])
+def test_dequantize_part_filled_and_unaligned(dt, n, k):
+    """Fewer values than a workgroup's 4096 (8192) and a remainder past it; a destination 2 / 4 bytes off the
+    16-byte grid gets the same bits as an aligned one and nothing around it is written; zeros keep their sign."""
+    import ctypes
+
+    from inference_amd import qmm
+    rng = np.random.default_rng(40 + n)
+    wq = orc.quantize(ORC[dt], (rng.standard_normal((n, k)) * 0.02).astype(np.float32))
+    qt = QTensor.from_ggml(wq, dt, (n, k), device=DEV)
+    ref = orc.dequantize(ORC[dt], wq, n * k).astype(np.float32)
+    for tag, tdt, bits, want in ((0, torch.float32, torch.int32, ref.view(np.int32)),
+                                 (1, torch.float16, torch.int16, ref.astype(np.float16).view(np.int16)),
+                                 (30, torch.bfloat16, torch.int16, bf16_rne(ref).view(np.int16))):
+        for off in (0, 1):
+            buf = torch.full((n * k + 16,), 7.0, dtype=tdt, device=DEV)
+            qmm._check(qmm.lib().qmm_qtensor_dequantize_to(qt.handle, buf.data_ptr() + off * buf.element_size(), tag,
+                                                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+            np.testing.assert_array_equal(buf[off:off + n * k].view(bits).cpu().numpy(), want)
+            assert (buf[:off] == 7.0).all() and (buf[off + n * k:] == 7.0).all()
