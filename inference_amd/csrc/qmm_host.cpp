@@ -816,7 +816,7 @@ static constexpr unsigned kS6StageBytes = 128 * 256 + 128 * 256 + 128 * 48 + 128
 static constexpr unsigned kSStageBytes = 128 * 256 + 128 * 128 + 128 * 16 + 128 * 4 + 128 * 48 + 128 * 48 + 128 * 80;
 // One LDS stage of the Q8_0 tile (mmqs8): activation rows, weight codes, f32
 // weight and activation block scales (the kernels' kS8Stage).
-static constexpr unsigned kS8StageBytes = 128 * 256 + 128 * 256 + 128 * 32 + 8 * 128 * 4;
+static constexpr unsigned kS8StageBytes = 128 * 256 + 128 * 256 + 128 * 16 + 128 * 16;
 static constexpr int kMmqBMRows = 64;             // and its M tile
 static void plan_splits(const Device* d, GemmPlan& p, int nbk) {
   const long long tiles = (long long)p.gx * p.gy;
@@ -934,7 +934,7 @@ static GemmPlan gemm_plan(const Device* d, const qmm_qtensor* w, int64_t m, bool
     p.threads = 512;
     p.lds = 2 * kS6StageBytes;
   } else if (fmt == kFmtQ80 && env(kEnvMmq8) == nullptr && (int)(2 * kS8StageBytes) <= d->max_lds) {
-    // Q8_0 default: mmqs8 (both operands straight into LDS, 128 x 128 tiles of eight waves, LDS 2 x 72 KB);
+    // Q8_0 default: mmqs8 (both operands straight into LDS, 128 x 128 tiles of eight waves, LDS 2 x 68 KB);
     // QMM_MMQ8=1 selects the first-generation tile
     snprintf(p.name, sizeof(p.name), "qmm_mmqs8_q8_0%s", dump ? "_dump" : "");
     p.gx = (unsigned)((N + 127) / 128);
@@ -1040,6 +1040,16 @@ static GemmPlan gemm_plan_fit(Device* d, const qmm_qtensor* w, int64_t m, bool d
   return p;
 }
 
+// y[m, n] (+)= the split partials [splits][m][n] at `part`, summed in split order.
+static int splitk_sum(Device* d, const float* part, int splits, int64_t m, int64_t n, float* y, int64_t ldy,
+                      int accumulate, hipStream_t s) {
+  // 16 bytes a thread where every row of the partials and of y starts on that grid
+  const bool v4 = n % 4 == 0 && ldy % 4 == 0 && ((uintptr_t)part | (uintptr_t)y) % 16 == 0;
+  int M = (int)m, N = (int)n, lo = (int)ldy;
+  void* args[] = {&part, &splits, &M, &N, &y, &lo, &accumulate};
+  return launch(d, v4 ? "qmm_splitk_sum4" : "qmm_splitk_sum", ceil_div(m * n / (v4 ? 4 : 1), 256), 256, 0, s, args);
+}
+
 // Prefill GEMM over activation planes at `ws` (see mmq_planes); `part` holds
 // part_bytes of scratch for split partials (a split plan that does not fit
 // runs as one split), which qmm_splitk_sum then adds into y.
@@ -1047,13 +1057,7 @@ static int gemm(Device* d, const qmm_qtensor* w, const uint8_t* ws, int64_t m, f
                 hipStream_t s, int accumulate, float* part, size_t part_bytes) {
   const GemmPlan p = gemm_plan_fit(d, w, m, dump != nullptr, part, part_bytes);
   QMM_TRY(gemm_launch(d, w, ws, m, p, y, ldy, dump, s, accumulate, part, part));
-  if (p.splits > 1) {
-    int M = (int)m, N = (int)w->n;
-    const float* pp = part;
-    int sp = p.splits, lo = (int)ldy;
-    void* a2[] = {&pp, &sp, &M, &N, &y, &lo, &accumulate};
-    QMM_TRY(launch(d, "qmm_splitk_sum", ceil_div((int64_t)M * N, 256), 256, 0, s, a2));
-  }
+  if (p.splits > 1) QMM_TRY(splitk_sum(d, part, p.splits, m, w->n, y, ldy, accumulate, s));
   return QMM_OK;
 }
 
@@ -1389,13 +1393,9 @@ static int matmul_targets(const GemvTarget* tg, int count, const float* x, int64
     MultiPlan mp;
     if (multi_plan(d, wl, count, m, &mp) && mp.bytes <= sb) {
       QMM_TRY(multi_launch(d, wl, mp, (const uint8_t*)ws, m, (uint8_t*)part, s));
-      for (int j = 0; j < count; ++j) {
-        int M = (int)m, N = (int)tg[j].w->n, sp = mp.splits[j], lo = (int)tg[j].ldy, acc = accumulate;
-        const float* pp = (const float*)((uint8_t*)part + mp.off[j]);
-        float* yy = tg[j].y;
-        void* a2[] = {&pp, &sp, &M, &N, &yy, &lo, &acc};
-        QMM_TRY(launch(d, "qmm_splitk_sum", ceil_div((int64_t)M * N, 256), 256, 0, s, a2));
-      }
+      for (int j = 0; j < count; ++j)
+        QMM_TRY(splitk_sum(d, (const float*)((uint8_t*)part + mp.off[j]), mp.splits[j], m, tg[j].w->n, tg[j].y,
+                           tg[j].ldy, accumulate, s));
       return QMM_OK;
     }
     for (int j = 0; j < count; ++j)
@@ -2561,13 +2561,7 @@ static int moe_gemm_planes(Device* d, const qmm_qtensor* const* w, int count, in
       void* args[] = {&wq, &q8, &dd, &ss, &yy, &N, &K, &ld, &E, &counts, &offsets, &kc, &ysplit};
       QMM_HIP(hipModuleLaunchKernel(f, (unsigned)((N + bn - 1) / bn), (unsigned)((max_rows + bm - 1) / bm),
                                     (unsigned)(experts * sp), threads, 1, 1, lds, s, args, nullptr));
-      if (sp > 1) {
-        const float* pp = part;
-        int spl = sp, M = (int)pairs, acc = 0;
-        float* yo = y[j];
-        void* a2[] = {&pp, &spl, &M, &N, &yo, &ld, &acc};
-        QMM_TRY(launch(d, "qmm_splitk_sum", ceil_div(pairs * N, 256), 256, 0, s, a2));
-      }
+      if (sp > 1) QMM_TRY(splitk_sum(d, part, sp, pairs, N, y[j], ld, 0, s));
     }
     return QMM_OK;
   }

@@ -576,7 +576,8 @@ extern "C" __global__ void __launch_bounds__(256) qmm_splitk_silu_mul_q8k_mmq(co
                      w, nb, k, q8, d, s, lane);
 }
 
-//   Q8_0: q8 int8 [m][k], d f32 [m][k/32] (the f16-rounded block scale)
+//   Q8_0: q8 int8 [m][k], d f32 [m][k/32] (the f16-rounded block scale); 333 x
+//   4096 takes 4.0 us (17 us when the block went through a scratch array)
 extern "C" __global__ void __launch_bounds__(256) qmm_quantize_q8_0_mmq(const float* __restrict__ x, long long ldx,
                                                                         int8_t* __restrict__ q8,
                                                                         float* __restrict__ d, int k, int m) {
@@ -586,13 +587,13 @@ extern "C" __global__ void __launch_bounds__(256) qmm_quantize_q8_0_mmq(const fl
   const bool valid = blk < (long long)m * nb;
   const long long bc = valid ? blk : 0;
   const int row = (int)(bc / nb), b = (int)(bc % nb), l = (int)(t & 7);
-  uint8_t tmp[qmm::kQ80Bytes];
-  qmm::q80_block(x + row * ldx + 32LL * b, tmp, l, valid);
+  const float* xs = x + row * ldx + 32LL * b + 4 * l;
+  const float e[4] = {xs[0], xs[1], xs[2], xs[3]};
+  uint16_t dh;
+  const uint32_t q = qmm::q80_lane(e, &dh);
   if (!valid) return;
-  const uint16_t* p = reinterpret_cast<const uint16_t*>(tmp);
-  reinterpret_cast<uint16_t*>(q8 + (size_t)row * k + 32 * b)[2 * l] = p[1 + 2 * l];
-  reinterpret_cast<uint16_t*>(q8 + (size_t)row * k + 32 * b)[2 * l + 1] = p[2 + 2 * l];
-  if (l == 0) d[bc] = qmm::h2f(p[0]);
+  reinterpret_cast<uint32_t*>(q8 + (size_t)row * k + 32 * b)[l] = q;
+  if (l == 0) d[bc] = qmm::h2f(dh);
 }
 
 #define QMM_MMQ_KERNEL(FMT, NAME)                                                                            \
@@ -1835,15 +1836,13 @@ __device__ __forceinline__ void mmqs6_q6k(const uint8_t* __restrict__ wq, const 
 // bytes (eight 32-blocks), so the activation rows and the weight codes both go
 // from global memory straight into LDS (global_load_lds, 16-byte chunks
 // swizzled by row / column as in mmqs); only the block scales pass through
-// registers (the weight's f16 d as f32 [col][8], the activation's f32 d
-// transposed to [block][row] so that four consecutive rows are one float4).
-// Per 32-block one int8 MFMA per 32 x 32 tile gives the block dot P exactly;
-// acc = fma(dw * dx, float(P), acc), the first-generation tile's sequence, so
-// the outputs equal its bits.
+// registers (f16 [col][8] and [row][8]). Per 32-block one int8 MFMA per 32 x 32
+// tile gives the block dot P exactly; acc = fma(dw * dx, float(P), acc), the
+// first-generation tile's sequence, so the outputs equal its bits.
 constexpr int kS8OffBq = kSBM * 256;             // weight codes [col][256], swizzled 16-byte slots
-constexpr int kS8OffDw = kS8OffBq + kSBN * 256;  // f32 d [col][8]
-constexpr int kS8OffDx = kS8OffDw + kSBN * 32;   // f32 d [block][row]
-constexpr int kS8Stage = kS8OffDx + 8 * kSBM * 4;
+constexpr int kS8OffDw = kS8OffBq + kSBN * 256;  // f16 d [col][8]
+constexpr int kS8OffDx = kS8OffDw + kSBN * 16;   // f16 d [row][8]
+constexpr int kS8Stage = kS8OffDx + kSBM * 16;
 
 struct SRegs8 {
   uint4 dw;   // t < 128: column t's eight f16 block scales
@@ -1885,69 +1884,98 @@ __device__ __forceinline__ void s8_load(SRegs8& R, uint8_t* stg, const int8_t* _
 __device__ __forceinline__ void s8_store(const SRegs8& R, uint8_t* buf) {
   const int t = threadIdx.x;
   if (t < 128) {
-    float* dw = reinterpret_cast<float*>(buf + kS8OffDw) + 8 * t;
-    const uint32_t v[4] = {R.dw.x, R.dw.y, R.dw.z, R.dw.w};
-    *reinterpret_cast<float4*>(dw) = make_float4(h2f(v[0]), h2f(v[0] >> 16), h2f(v[1]), h2f(v[1] >> 16));
-    *reinterpret_cast<float4*>(dw + 4) = make_float4(h2f(v[2]), h2f(v[2] >> 16), h2f(v[3]), h2f(v[3] >> 16));
+    *reinterpret_cast<uint4*>(buf + kS8OffDw + 16 * t) = R.dw;
   } else if (t < 384) {
-    const int i = t - 128, row = i >> 1, q = i & 1;
-    float* dx = reinterpret_cast<float*>(buf + kS8OffDx);
-    dx[(4 * q) * kSBM + row] = R.dx.x;
-    dx[(4 * q + 1) * kSBM + row] = R.dx.y;
-    dx[(4 * q + 2) * kSBM + row] = R.dx.z;
-    dx[(4 * q + 3) * kSBM + row] = R.dx.w;
+    // (the f32 scales are f16 values: exact)
+    *reinterpret_cast<uint2*>(buf + kS8OffDx + 8 * (t - 128)) =
+        make_uint2((uint32_t)f2h(R.dx.x) | (uint32_t)f2h(R.dx.y) << 16, (uint32_t)f2h(R.dx.z) | (uint32_t)f2h(R.dx.w) << 16);
   }
 }
 
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+
 // One K step from stage `buf`. Wave w owns rows 32 (w & 3) .. + 32 and the
-// two 32-column tiles of columns 64 (w >> 2) .. + 64, so a lane's 16 outputs
-// per tile share their rows across both tiles: per 32-block c the lane reads
-// its rows' 16 activation scales once (four float4 from the [block][row]
-// layout) and one weight scale per tile. Per tile j, P = the MFMA block dot,
-// acc += (dw * dx) * P. DUMP: every block dot.
+// two 32-column tiles of columns 64 (w >> 2) .. + 64. Per 32-block c and tile:
+//   P = the block dot (one int8 MFMA), accumulated onto 1.5 * 2^23 as an integer: its
+//       bits are then the float 1.5 * 2^23 + P (|P| < 2^20), and one subtraction
+//       gives float(P), at the f32 rate of two cycles an instruction where a
+//       conversion takes four;
+//   S = dx * dw of every output, one f16 MFMA with block c's scales in its k
+//       slot and zeros elsewhere: both are f16 values, so the products are exact
+//       (the f32 products of the first-generation tile), and neither a multiply
+//       per output nor an LDS read of the rows' scales per block is left;
+//   acc = fma(S, P, acc), the first-generation tile's sequence and bits.
+// Bound by VALU issue: two f32 instructions per output and block, beside two
+// MFMAs that each hold the SIMD's issue for 16 cycles. 512 x 14336 x 4096: 112 us
+// (132 us with a conversion and two multiplies per output and block); 333 x 4096 x
+// 4096 unsplit 47 us (59 us).
+// DUMP: every block dot.
 template <bool DUMP>
 __device__ __forceinline__ void mmqs8_step(const uint8_t* __restrict__ buf, f32x16 (&acc)[2], int wm, int wn, int r,
                                            int h, int m0, int n0, int M, int N, int nbw, int kb,
                                            int* __restrict__ dump) {
 #pragma clang fp contract(off)
-  i32x16 zero;
+  constexpr float kMagic = 12582912.0f;  // 1.5 * 2^23
+  i32x16 magic;
+  f32x16 zero;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) zero[j] = 0;
+  for (int j = 0; j < 16; ++j) {
+    magic[j] = __builtin_bit_cast(int, kMagic);
+    zero[j] = 0.0f;
+  }
   const int arow = 32 * wm + r, sa = r & 15;
   const int8_t* A = reinterpret_cast<const int8_t*>(buf) + 256 * arow;
   const int8_t* B = reinterpret_cast<const int8_t*>(buf + kS8OffBq) + 256 * (64 * wn + r);
-  const float* DW = reinterpret_cast<const float*>(buf + kS8OffDw) + 8 * (64 * wn + r);
-  const float* DX = reinterpret_cast<const float*>(buf + kS8OffDx) + 32 * wm + 4 * h;
-  // two blocks at a time (fully unrolled, the compiler hoists every MFMA of
-  // the step ahead of the epilogues and spills)
-#pragma unroll 2
-  for (int c = 0; c < 8; ++c) {
-    const int slot = 2 * c + h;  // 16-byte chunk of this lane half
-    const i8x16 a = *reinterpret_cast<const i8x16*>(A + 16 * (slot ^ sa));
-    float dxs[16];
+  // k slots 4 h .. 4 h + 3 of the scale product: blocks 4 h .. 4 h + 3
+  const uint2 dx = *reinterpret_cast<const uint2*>(buf + kS8OffDx + 16 * arow + 8 * h);
+  uint2 dw[2];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const float4 dx = *reinterpret_cast<const float4*>(DX + c * kSBM + 8 * g);
-      dxs[4 * g] = dx.x;
-      dxs[4 * g + 1] = dx.y;
-      dxs[4 * g + 2] = dx.z;
-      dxs[4 * g + 3] = dx.w;
+  for (int j = 0; j < 2; ++j)
+    dw[j] = *reinterpret_cast<const uint2*>(buf + kS8OffDw + 16 * (64 * wn + 32 * j + r) + 8 * h);
+  auto only = [&](uint2 v, int c) {  // block c's scale in its slot, zeros in the others
+    const uint32_t m = h == (c >> 2) ? ((c & 1) ? 0xffff0000u : 0x0000ffffu) : 0u;
+    return __builtin_bit_cast(f16x4, make_uint2((c & 2) ? 0u : v.x & m, (c & 2) ? v.y & m : 0u));
+  };
+  // (block, tile) pairs in order: pair i + 1's MFMAs run under pair i's epilogue,
+  // its operand reads under the one before (the barriers keep the compiler from
+  // hoisting every MFMA of the step ahead of the epilogues)
+  i8x16 a, b;
+  auto fetch = [&](int i) {
+    const int slot = 2 * (i >> 1) + h;  // 16-byte chunk of this lane half
+    if ((i & 1) == 0) a = *reinterpret_cast<const i8x16*>(A + 16 * (slot ^ sa));
+    // the swizzle of column 64 wn + 32 j + r is r & 15
+    b = *reinterpret_cast<const i8x16*>(B + 256 * 32 * (i & 1) + 16 * (slot ^ sa));
+  };
+  i32x16 P[2];
+  f32x16 S[2];
+  fetch(0);
+#pragma unroll
+  for (int i = 0; i <= 16; ++i) {
+    if (i < 16) {
+      P[i & 1] = mfma_i8(a, b, magic);
+      S[i & 1] = __builtin_amdgcn_mfma_f32_32x32x8f16(only(dx, i >> 1), only(dw[i & 1], i >> 1), zero, 0, 0, 0);
+      asm volatile("" : "+v"(P[i & 1]), "+v"(S[i & 1]));  // issued here, ahead of the epilogue below
+      if (i < 15) fetch(i + 1);
     }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      // columns 32 j + r: the swizzle of column 64 wn + 32 j + r is r & 15
-      const i8x16 b = *reinterpret_cast<const i8x16*>(B + 256 * 32 * j + 16 * (slot ^ sa));
-      const float dwc = DW[256 * j + c];
-      const i32x16 P = mfma_i8(a, b, zero);
+    if (i > 0) {
+      const int j = (i - 1) & 1;
+      f32x16 pf;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        acc[j][e] = __builtin_fmaf(dwc * dxs[e], (float)P[e], acc[j][e]);
+        const int p = P[j][e];  // (a copy: bit_cast of a vector element itself takes element 0)
+        pf[e] = __builtin_bit_cast(float, p) - kMagic;
         if (DUMP) {
           const int row = m0 + 32 * wm + 8 * (e >> 2) + 4 * h + (e & 3), col = n0 + 64 * wn + 32 * j + r;
-          if (row < M && col < N) dump[((size_t)row * N + col) * nbw + 8 * kb + c] = P[e];
+          if (row < M && col < N)
+            dump[((size_t)row * N + col) * nbw + 8 * kb + ((i - 1) >> 1)] = p - __builtin_bit_cast(int, kMagic);
         }
       }
+      asm volatile("" : "+v"(pf));  // sixteen independent instructions, then sixteen more
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[j][e] = __builtin_fmaf(S[j][e], pf[e], acc[j][e]);
+      asm volatile("" : "+v"(acc[j]));  // here, not sunk past the step's other MFMAs
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -2131,16 +2159,47 @@ QMM_MMQ2_KERNEL(64, 128)
 QMM_MMQ2_KERNEL(64, 64)
 
 // Split-K sum: y[m, n] (+)= part[0][m, n] + ... + part[splits - 1][m, n], in
-// split order (partials [splits][M][N], row stride N).
+// split order (partials [splits][M][N], row stride N). Bound by memory; a
+// thread sums V neighbouring outputs (four where rows and pointers allow
+// 16-byte accesses, which the host checks), four splits' loads in flight.
+// 333 x 4096 over 2 splits: 8.2 us, 10.0 us one output a thread.
+namespace qmm {
+template <int V>
+__device__ __forceinline__ void splitk_sum(const float* __restrict__ part, int splits, int M, int N,
+                                           float* __restrict__ y, int ldy, int accumulate) {
+  struct __attribute__((aligned(4 * V))) Vec {
+    float v[V];
+  };
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  const unsigned nv = (unsigned)N / V;
+  if (i >= (long long)M * nv) return;
+  const int m = (int)(i / nv), n = V * (int)(i - (long long)m * nv);
+  const size_t plane = (size_t)M * N;
+  const float* p = part + (size_t)V * i;
+  Vec s = *reinterpret_cast<const Vec*>(p);
+#pragma unroll 4
+  for (int k = 1; k < splits; ++k) {
+    const Vec x = *reinterpret_cast<const Vec*>(p + k * plane);
+#pragma unroll
+    for (int e = 0; e < V; ++e) s.v[e] += x.v[e];
+  }
+  Vec* yp = reinterpret_cast<Vec*>(y + (size_t)m * ldy + n);
+  if (accumulate) {
+    const Vec o = *yp;
+#pragma unroll
+    for (int e = 0; e < V; ++e) s.v[e] = o.v[e] + s.v[e];
+  }
+  *yp = s;
+}
+}  // namespace qmm
+
 extern "C" __global__ void __launch_bounds__(256) qmm_splitk_sum(const float* __restrict__ part, int splits, int M,
                                                                  int N, float* __restrict__ y, int ldy,
                                                                  int accumulate) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long long)M * N) return;
-  const int m = (int)(i / N), n = (int)(i - (long long)m * N);
-  const size_t plane = (size_t)M * N;
-  float s = part[i];
-  for (int k = 1; k < splits; ++k) s += part[i + k * plane];
-  float* yp = y + (size_t)m * ldy + n;
-  *yp = accumulate ? *yp + s : s;
+  qmm::splitk_sum<1>(part, splits, M, N, y, ldy, accumulate);
+}
+extern "C" __global__ void __launch_bounds__(256) qmm_splitk_sum4(const float* __restrict__ part, int splits, int M,
+                                                                  int N, float* __restrict__ y, int ldy,
+                                                                  int accumulate) {
+  qmm::splitk_sum<4>(part, splits, M, N, y, ldy, accumulate);
 }
