@@ -1015,7 +1015,9 @@ static int gemm_launch(Device* d, const qmm_qtensor* w, const uint8_t* ws, int64
   long long ysplit = split ? (long long)M * N : 0;
   void* args[] = {&wq, &q8, &dd, &ss, &yy, &M, &N, &K, &ld, &dp, &acc, &remap, &kc, &ysplit};
   hipFunction_t f;
-  QMM_TRY(kernel(d, p.name, &f));
+  // Q6_K up to 64 rows: the tile that skips its empty row tiles (the same bits; see mmqs6_q6k_at)
+  const bool s6 = m <= 64 && strcmp(p.name, "qmm_mmqs6_q6k") == 0;
+  QMM_TRY(kernel(d, s6 ? "qmm_mmqs6_q6k_short" : p.name, &f));
   QMM_HIP(hipModuleLaunchKernel(f, p.gx, p.gy, (unsigned)p.splits, p.threads, 1, 1, p.lds, s, args, nullptr));
   return QMM_OK;
 }

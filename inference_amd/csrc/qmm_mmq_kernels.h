@@ -1072,7 +1072,8 @@ __device__ __forceinline__ void mmq4_q4k(const uint8_t* __restrict__ wq, const i
 //   * workgroup tile 128 x 128, eight waves (two per SIMD, so one wave's
 //     VALU epilogue and LDS waits overlap the other's MFMAs), two along M and
 //     four along N; a wave owns 64 rows (two M tiles) x 32 columns, so a
-//     column's operand products are formed once per K step for two tiles;
+//     column's operand products are formed once per K step for two tiles; an M
+//     tile past the last row is skipped;
 //     the mins MFMAs and the d-term multiply-adds share one f32 accumulator;
 //   * staging: two LDS stages; the next step's activation rows and weight
 //     quants go from global memory straight into the other stage
@@ -1087,7 +1088,8 @@ __device__ __forceinline__ void mmq4_q4k(const uint8_t* __restrict__ wq, const i
 //     header and form B' and the split-scale multipliers as packed 16-bit
 //     pairs; threads 128..255 load row t - 128's scale and sums and form A'
 //     (waves 0, 1 and 2, 3: the staging arithmetic lands on all four SIMDs,
-//     wave w running on SIMD w % 4). A' / B' / multiplier rows sit at odd
+//     wave w running on SIMD w % 4, and on the older wave of each, which
+//     issues first: on waves 4..7 a K step took 14% longer). A' / B' / multiplier rows sit at odd
 //     multiples of 16 bytes (conflict-free 16-byte access).
 // DUMP instantiations also compute ism exactly (two zero-padded int8 MFMAs)
 // and write the integer block dots, which equal mmq2's.
@@ -1110,6 +1112,11 @@ template <bool DUMP>
 struct SLayout {
   static constexpr int kStage = kSOffSum + (DUMP ? kSBM * 16 : 0);
   static constexpr int kBytes = 2 * kStage;
+};
+
+template <int V>
+struct Int {
+  static constexpr int value = V;
 };
 
 struct SRegs {
@@ -1249,6 +1256,7 @@ __device__ __forceinline__ i8x16 bytes_times4p(uint4 v, uint32_t s2) {
 
 // The integer part of one K step of mmqs from LDS stage `buf`: accl / acch =
 // the split-scale MFMA sums (isd = accl + 8 acch).
+template <int NT>
 __device__ __forceinline__ void mmqs_mfma(const uint8_t* __restrict__ buf, i32x16 (&accl)[kSTM],
                                           i32x16 (&acch)[kSTM], int wm, int r, int h, int bcol) {
   i32x16 zero;
@@ -1274,22 +1282,22 @@ __device__ __forceinline__ void mmqs_mfma(const uint8_t* __restrict__ buf, i32x1
     const i8x16 bh0 = bytes_times4p(blo, pick(sh4, 2 * c2));
     const i8x16 bl1 = bytes_times4p(bhi, pick(sl4, 2 * c2 + 1));
     const i8x16 bh1 = bytes_times4p(bhi, pick(sh4, 2 * c2 + 1));
-    i8x16 a0[kSTM], a1[kSTM];
+    i8x16 a0[NT], a1[NT];
 #pragma unroll
-    for (int i = 0; i < kSTM; ++i) {
+    for (int i = 0; i < NT; ++i) {
       const int8_t* ar = A + 256 * (arow0 + 32 * i);
       a0[i] = *reinterpret_cast<const i8x16*>(ar + 16 * ((4 * c2 + h) ^ sa));
       a1[i] = *reinterpret_cast<const i8x16*>(ar + 16 * ((4 * c2 + 2 + h) ^ sa));
     }
     // chains on one accumulator four MFMAs apart
 #pragma unroll
-    for (int i = 0; i < kSTM; ++i) accl[i] = mfma_i8(a0[i], bl0, c2 == 0 ? zero : accl[i]);
+    for (int i = 0; i < NT; ++i) accl[i] = mfma_i8(a0[i], bl0, c2 == 0 ? zero : accl[i]);
 #pragma unroll
-    for (int i = 0; i < kSTM; ++i) acch[i] = mfma_i8(a0[i], bh0, c2 == 0 ? zero : acch[i]);
+    for (int i = 0; i < NT; ++i) acch[i] = mfma_i8(a0[i], bh0, c2 == 0 ? zero : acch[i]);
 #pragma unroll
-    for (int i = 0; i < kSTM; ++i) accl[i] = mfma_i8(a1[i], bl1, accl[i]);
+    for (int i = 0; i < NT; ++i) accl[i] = mfma_i8(a1[i], bl1, accl[i]);
 #pragma unroll
-    for (int i = 0; i < kSTM; ++i) acch[i] = mfma_i8(a1[i], bh1, acch[i]);
+    for (int i = 0; i < NT; ++i) acch[i] = mfma_i8(a1[i], bh1, acch[i]);
   }
 }
 
@@ -1297,6 +1305,7 @@ __device__ __forceinline__ void mmqs_mfma(const uint8_t* __restrict__ buf, i32x1
 // the bf16 matrix cores (lane half h supplies K half h of each MFMA: pieces
 // [a1 | a2] x [b1 | b1], [a1 | a2] x [b2 | b2], [a1 | a3] x [b3 | b1]) and
 // acc += (dx * d) * isd.
+template <int NT>
 __device__ __forceinline__ void mmqs_epi(const uint8_t* __restrict__ buf, const i32x16 (&accl)[kSTM],
                                          const i32x16 (&acch)[kSTM], f32x16 (&acc)[kSTM], int wm, int r, int h,
                                          int bcol) {
@@ -1308,7 +1317,7 @@ __device__ __forceinline__ void mmqs_epi(const uint8_t* __restrict__ buf, const 
   const bf16x8 b2 = *reinterpret_cast<const bf16x8*>(bmp + 16);
   const bf16x8 b31 = *reinterpret_cast<const bf16x8*>(bmp + (h == 0 ? 32 : 0));
 #pragma unroll
-  for (int i = 0; i < kSTM; ++i) {
+  for (int i = 0; i < NT; ++i) {
     const uint8_t* amp = buf + kSOffAm + kSHalf * (arow0 + 32 * i);
     const bf16x8 a12 = *reinterpret_cast<const bf16x8*>(amp + 16 * h);
     const bf16x8 a13 = *reinterpret_cast<const bf16x8*>(amp + 32 * h);
@@ -1317,7 +1326,7 @@ __device__ __forceinline__ void mmqs_epi(const uint8_t* __restrict__ buf, const 
     acc[i] = mfma_bf16(a13, b31, acc[i]);
   }
 #pragma unroll
-  for (int i = 0; i < kSTM; ++i) {
+  for (int i = 0; i < NT; ++i) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const float4 dx = *reinterpret_cast<const float4*>(DX + 64 * wm + 32 * i + 8 * g + 4 * h);
@@ -1341,7 +1350,7 @@ __device__ __forceinline__ void mmqs_step_dump(const uint8_t* __restrict__ buf, 
 #pragma unroll
   for (int j = 0; j < 16; ++j) zero[j] = 0;
   i32x16 accl[kSTM], acch[kSTM];
-  mmqs_mfma(buf, accl, acch, wm, r, h, bcol);
+  mmqs_mfma<kSTM>(buf, accl, acch, wm, r, h, bcol);
   const int arow0 = 64 * wm + r;
   const float* DX = reinterpret_cast<const float*>(buf + kSOffDx);
   const uint4 hd = *reinterpret_cast<const uint4*>(buf + kSOffHd + 16 * bcol);
@@ -1369,6 +1378,15 @@ __device__ __forceinline__ void mmqs_step_dump(const uint8_t* __restrict__ buf, 
   }
 }
 
+// How many of a wave's two row tiles (rows 64 wm and 64 wm + 32 of the
+// workgroup's) hold rows of the product. The others' products would be padding,
+// so a wave runs the K loop of its count; consecutive tiles, because a wave forms
+// the column operands once for both.
+__device__ __forceinline__ int rows_filled(int M, int m0, int wm) {
+  const int left = M - m0 - 64 * wm;
+  return left > 32 ? 2 : left > 0 ? 1 : 0;
+}
+
 // K steps [kb0, kb1) of the 128 x 128 tile at (m0, n0) into acc (zeroed
 // first): the staging / MFMA loop of one tile. Ends with a barrier after the
 // last step, so the LDS stages are free for the next call.
@@ -1380,9 +1398,9 @@ __device__ __forceinline__ void mmqs_run(const uint8_t* __restrict__ wq, const i
   using Lay = SLayout<DUMP>;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int nbk = K / 256;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 31, h = lane >> 5;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave >> 2, wn = wave & 3;  // (wave w runs on SIMD w % 4: one of either half on each)
   const int bcol = 32 * wn + r;  // this lane's column in the workgroup tile
   const int col = n0 + bcol;
 
@@ -1399,21 +1417,33 @@ __device__ __forceinline__ void mmqs_run(const uint8_t* __restrict__ wq, const i
   s_store<DUMP>(R, lds);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
-  i32x16 accl[kSTM], acch[kSTM];
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const uint8_t* cur = lds + ((kb - kb0) & 1) * Lay::kStage;
-    uint8_t* nxt = lds + ((kb + 1 - kb0) & 1) * Lay::kStage;
-    if (kb + 1 < kb1) s_load(R, nxt, xq, xd, xs, wq, M, N, K, m0, n0, kb + 1);
-    if constexpr (DUMP) {
-      mmqs_step_dump(cur, acc, wm, r, h, bcol, m0, col, M, N, nbk, kb, dump);
-    } else {
-      mmqs_mfma(cur, accl, acch, wm, r, h, bcol);
-      mmqs_epi(cur, accl, acch, acc, wm, r, h, bcol);
+  // one copy of the loop per count of filled row tiles (a branch inside one loop cost whole tiles 5%: the
+  // staging no longer ran under their last MFMAs); every copy meets the same barriers
+  auto loop = [&](auto nt) {
+    constexpr int NT = decltype(nt)::value;
+    i32x16 accl[kSTM], acch[kSTM];
+    for (int kb = kb0; kb < kb1; ++kb) {
+      const uint8_t* cur = lds + ((kb - kb0) & 1) * Lay::kStage;
+      uint8_t* nxt = lds + ((kb + 1 - kb0) & 1) * Lay::kStage;
+      if (kb + 1 < kb1) s_load(R, nxt, xq, xd, xs, wq, M, N, K, m0, n0, kb + 1);
+      if constexpr (DUMP) {
+        mmqs_step_dump(cur, acc, wm, r, h, bcol, m0, col, M, N, nbk, kb, dump);
+      } else if constexpr (NT > 0) {
+        mmqs_mfma<NT>(cur, accl, acch, wm, r, h, bcol);
+        mmqs_epi<NT>(cur, accl, acch, acc, wm, r, h, bcol);
+      }
+      if (kb + 1 < kb1) s_store<DUMP>(R, nxt);
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+      __syncthreads();
     }
-    if (kb + 1 < kb1) s_store<DUMP>(R, nxt);
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-    __syncthreads();
-  }
+  };
+  const int filled = DUMP ? 2 : rows_filled(M, m0, wm);
+  if (filled == 2)
+    loop(Int<2>{});
+  else if (filled == 1)
+    loop(Int<1>{});
+  else
+    loop(Int<0>{});
 }
 
 // acc of the tile at (m0, n0) -> y (rows < M, columns < N; added to y when
@@ -1423,7 +1453,7 @@ __device__ __forceinline__ void mmqs_store(const f32x16 (&acc)[kSTM], float* __r
                                            int m0, int n0, int accumulate) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r = lane & 31, h = lane >> 5;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave >> 2, wn = wave & 3;
   const int col = n0 + 32 * wn + r;
 #pragma unroll
   for (int i = 0; i < kSTM; ++i)
@@ -1705,6 +1735,7 @@ __device__ __forceinline__ void s6_store(const SRegs6& R, uint8_t* buf) {
 
 // One K step's digit sums from stage `buf`: acc[d][i] = MFMA-sum over the
 // step of x (row tile i) and d_d * q (the lane's column).
+template <int NT>
 __device__ __forceinline__ void mmqs6_mfma(const uint8_t* __restrict__ buf, i32x16 (&acc)[3][kSTM], int wm, int r,
                                            int h, int bcol) {
   i32x16 zero;
@@ -1727,9 +1758,9 @@ __device__ __forceinline__ void mmqs6_mfma(const uint8_t* __restrict__ buf, i32x
       ev[k] = bw[k] & 0x00ff00ffu;
       od[k] = (bw[k] >> 8) & 0x00ff00ffu;
     }
-    i8x16 a[kSTM];
+    i8x16 a[NT];
 #pragma unroll
-    for (int i = 0; i < kSTM; ++i)
+    for (int i = 0; i < NT; ++i)
       a[i] = *reinterpret_cast<const i8x16*>(A + 256 * (arow0 + 32 * i) + 16 * ((2 * c + h) ^ sa));
     const int sh = 8 * (2 * (c & 1) + h);  // byte (2 c + h) of the digit rows: dword c / 2
 #pragma unroll
@@ -1745,14 +1776,14 @@ __device__ __forceinline__ void mmqs6_mfma(const uint8_t* __restrict__ buf, i32x
       }
       const i8x16 bd = as_i8x16(make_uint4(w[0], w[1], w[2], w[3]));
 #pragma unroll
-      for (int i = 0; i < kSTM; ++i) acc[d][i] = mfma_i8(a[i], bd, c == 0 ? zero : acc[d][i]);
+      for (int i = 0; i < NT; ++i) acc[d][i] = mfma_i8(a[i], bd, c == 0 ? zero : acc[d][i]);
     }
   }
 }
 
 // acc = fma(dx, d * isum, acc) per output (isum = D0 + 8 D1 + 64 D2); DUMP:
 // every block's isum.
-template <bool DUMP>
+template <int NT, bool DUMP>
 __device__ __forceinline__ void mmqs6_epi(const uint8_t* __restrict__ buf, const i32x16 (&dsum)[3][kSTM],
                                           f32x16 (&acc)[kSTM], int wm, int r, int h, int bcol, int m0, int col,
                                           int M, int N, int nbk, int kb, int* __restrict__ dump) {
@@ -1760,7 +1791,7 @@ __device__ __forceinline__ void mmqs6_epi(const uint8_t* __restrict__ buf, const
   const float* DX = reinterpret_cast<const float*>(buf + kS6OffDx);
   const float dw = reinterpret_cast<const float*>(buf + kS6OffDw)[bcol];
 #pragma unroll
-  for (int i = 0; i < kSTM; ++i) {
+  for (int i = 0; i < NT; ++i) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const float4 dx = *reinterpret_cast<const float4*>(DX + 64 * wm + 32 * i + 8 * g + 4 * h);
@@ -1783,7 +1814,10 @@ __device__ __forceinline__ void mmqs6_epi(const uint8_t* __restrict__ buf, const
 
 // The 128 x 128 tile at (m0, n0), K steps [kb0, kb1), into y.
 // wd: the weight's separated f16 d per block (row-major, K / 256 per row).
-template <bool DUMP>
+// SHORT: row tiles past the last row are skipped. The branch costs a whole tile 3%
+// (in copies of the loop, as in mmqs_run, it spills), so the host takes it where
+// no tile is whole: 14336 x 4096, 9 rows 45 us against 74, 64 rows 66 against 74.
+template <bool DUMP, bool SHORT = false>
 __device__ __forceinline__ void mmqs6_q6k_at(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd,
                                              const int8_t* __restrict__ xq, const float* __restrict__ xd,
                                              float* __restrict__ y, int M, int N, int K, int ldy,
@@ -1791,9 +1825,9 @@ __device__ __forceinline__ void mmqs6_q6k_at(const uint8_t* __restrict__ wq, con
                                              int kb1) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int nbk = K / 256;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 31, h = lane >> 5;
-  const int wm = wave & 1, wn = wave >> 1;
+  const int wm = wave >> 2, wn = wave & 3;
   const int bcol = 32 * wn + r;
   const int col = n0 + bcol;
   f32x16 acc[kSTM];
@@ -1806,13 +1840,19 @@ __device__ __forceinline__ void mmqs6_q6k_at(const uint8_t* __restrict__ wq, con
   s6_store(R, lds);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
+  const int filled = SHORT ? rows_filled(M, m0, wm) : 2;
   for (int kb = kb0; kb < kb1; ++kb) {
     const uint8_t* cur = lds + ((kb - kb0) & 1) * kS6Stage;
     uint8_t* nxt = lds + ((kb + 1 - kb0) & 1) * kS6Stage;
     if (kb + 1 < kb1) s6_load(R, nxt, xq, xd, wq, wd, M, N, K, m0, n0, kb + 1);
     i32x16 dsum[3][kSTM];
-    mmqs6_mfma(cur, dsum, wm, r, h, bcol);
-    mmqs6_epi<DUMP>(cur, dsum, acc, wm, r, h, bcol, m0, col, M, N, nbk, kb, dump);
+    if (filled == 2) {
+      mmqs6_mfma<2>(cur, dsum, wm, r, h, bcol);
+      mmqs6_epi<2, DUMP>(cur, dsum, acc, wm, r, h, bcol, m0, col, M, N, nbk, kb, dump);
+    } else if (filled == 1) {
+      mmqs6_mfma<1>(cur, dsum, wm, r, h, bcol);
+      mmqs6_epi<1, DUMP>(cur, dsum, acc, wm, r, h, bcol, m0, col, M, N, nbk, kb, dump);
+    }
     if (kb + 1 < kb1) s6_store(R, nxt);
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     __syncthreads();
@@ -1820,14 +1860,14 @@ __device__ __forceinline__ void mmqs6_q6k_at(const uint8_t* __restrict__ wq, con
   mmqs_store(acc, y, M, N, ldy, m0, n0, accumulate);
 }
 
-template <bool DUMP>
+template <bool DUMP, bool SHORT = false>
 __device__ __forceinline__ void mmqs6_q6k(const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd,
                                           const int8_t* __restrict__ xq, const float* __restrict__ xd,
                                           float* __restrict__ y, int M, int N, int K, int ldy,
                                           int* __restrict__ dump, int accumulate, int remap, int kb0, int kb1) {
   int mt, nt;
   gemm_tile(remap, mt, nt);
-  mmqs6_q6k_at<DUMP>(wq, wd, xq, xd, y, M, N, K, ldy, dump, accumulate, mt * kSBM, nt * kSBN, kb0, kb1);
+  mmqs6_q6k_at<DUMP, SHORT>(wq, wd, xq, xd, y, M, N, K, ldy, dump, accumulate, mt * kSBM, nt * kSBN, kb0, kb1);
 }
 
 // Q8_0 prefill GEMM on the mmqs scaffold (mmqs8_q8_0): 128 x 128 tiles of
@@ -1894,8 +1934,8 @@ __device__ __forceinline__ void s8_store(const SRegs8& R, uint8_t* buf) {
 
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
-// One K step from stage `buf`. Wave w owns rows 32 (w & 3) .. + 32 and the
-// two 32-column tiles of columns 64 (w >> 2) .. + 64. Per 32-block c and tile:
+// One K step from stage `buf`. Wave w owns rows 32 (w >> 1) .. + 32 and the
+// two 32-column tiles of columns 64 (w & 1) .. + 64. Per 32-block c and tile:
 //   P = the block dot (one int8 MFMA), accumulated onto 1.5 * 2^23 as an integer: its
 //       bits are then the float 1.5 * 2^23 + P (|P| < 2^20), and one subtraction
 //       gives float(P), at the f32 rate of two cycles an instruction where a
@@ -1990,9 +2030,9 @@ __device__ __forceinline__ void mmqs8_q8_0(const uint8_t* __restrict__ wq, const
   gemm_tile(remap, mt, nt);
   const int m0 = mt * kSBM, n0 = nt * kSBN;
   const int nbw = K / 32;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 31, h = lane >> 5;
-  const int wm = wave & 3, wn = wave >> 2;
+  const int wm = wave >> 1, wn = wave & 1;
   f32x16 acc[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
@@ -2003,15 +2043,22 @@ __device__ __forceinline__ void mmqs8_q8_0(const uint8_t* __restrict__ wq, const
   s8_store(R, lds);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
   __syncthreads();
-  for (int kb = kb0; kb < kb1; ++kb) {
-    const uint8_t* cur = lds + ((kb - kb0) & 1) * kS8Stage;
-    uint8_t* nxt = lds + ((kb + 1 - kb0) & 1) * kS8Stage;
-    if (kb + 1 < kb1) s8_load(R, nxt, xq, xd, wq, wd, M, N, K, m0, n0, kb + 1);
-    mmqs8_step<DUMP>(cur, acc, wm, wn, r, h, m0, n0, M, N, nbw, kb, dump);
-    if (kb + 1 < kb1) s8_store(R, nxt);
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-    __syncthreads();
-  }
+  auto loop = [&](auto nt) {  // a wave without rows of the product only stages
+    constexpr int NT = decltype(nt)::value;
+    for (int kb = kb0; kb < kb1; ++kb) {
+      const uint8_t* cur = lds + ((kb - kb0) & 1) * kS8Stage;
+      uint8_t* nxt = lds + ((kb + 1 - kb0) & 1) * kS8Stage;
+      if (kb + 1 < kb1) s8_load(R, nxt, xq, xd, wq, wd, M, N, K, m0, n0, kb + 1);
+      if constexpr (NT > 0) mmqs8_step<DUMP>(cur, acc, wm, wn, r, h, m0, n0, M, N, nbw, kb, dump);
+      if (kb + 1 < kb1) s8_store(R, nxt);
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+      __syncthreads();
+    }
+  };
+  if (m0 + 32 * wm < M)
+    loop(Int<1>{});
+  else
+    loop(Int<0>{});
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int col = n0 + 64 * wn + 32 * j + r;
@@ -2042,7 +2089,7 @@ __device__ __forceinline__ void mmqs8_q8_0(const uint8_t* __restrict__ wq, const
 QMM_MMQS8_KERNEL(, false)
 QMM_MMQS8_KERNEL(_dump, true)
 
-#define QMM_MMQS6_KERNEL(SUFFIX, DUMP)                                                                         \
+#define QMM_MMQS6_KERNEL(SUFFIX, DUMP, SHORT)                                                                  \
   extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))                 \
       qmm_mmqs6_q6k##SUFFIX(const uint8_t* __restrict__ wq, const int8_t* __restrict__ xq,                     \
                             const float* __restrict__ xd, const int16_t* __restrict__ xs,                      \
@@ -2050,11 +2097,12 @@ QMM_MMQS8_KERNEL(_dump, true)
                             int accumulate, int remap, int kc, long long ysplit) {                             \
     (void)xs;                                                                                                  \
     const qmm::KRange kr = qmm::split_range(K, kc);                                                            \
-    qmm::mmqs6_q6k<DUMP>(wq, qmm::split_scales<qmm::kFmtQ6K>(wq, N, K), xq, xd, y + blockIdx.z * ysplit, M, N, \
-                         K, ldy, dump, accumulate, remap, kr.kb0, kr.kb1);                                     \
+    qmm::mmqs6_q6k<DUMP, SHORT>(wq, qmm::split_scales<qmm::kFmtQ6K>(wq, N, K), xq, xd, y + blockIdx.z * ysplit, \
+                         M, N, K, ldy, dump, accumulate, remap, kr.kb0, kr.kb1);                                     \
   }
-QMM_MMQS6_KERNEL(, false)
-QMM_MMQS6_KERNEL(_dump, true)
+QMM_MMQS6_KERNEL(, false, false)
+QMM_MMQS6_KERNEL(_short, false, true)
+QMM_MMQS6_KERNEL(_dump, true, false)
 
 // Up to three Q4_K / Q6_K weights of one K over the same activation planes in
 // one launch (the prefill's q / k / v), each split over K into f32 partials:
