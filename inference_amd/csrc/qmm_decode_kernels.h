@@ -158,7 +158,19 @@ extern "C" __global__ void qmm_prefill_splitk_rope_kv(const float* __restrict__ 
 // online per row, a batch of positions at a time (m = running max,
 // l = sum exp(s - m), o = sum exp(s - m) v). The next batch's k/v rows are
 // loaded while the current batch is scored. The rows' states are combined
-// through LDS.
+// through LDS. The exponentials are 2^(s log2 e - m log2 e) with one rounding
+// each; the states and records carry m log2 e, the value that was subtracted.
+//
+// What bounds it: VALU issue (dots and weighted sums of G heads over every
+// position) up to a few thousand positions on half the CUs, above a fixed ~8 us
+// of dependent round trips (position, rows, record, counter, records). 32 / 8
+// heads of 128 at 3001 positions 12.9 us, 17.2 with a library exponential and
+// separate multiplies and additions; 32 chunks instead of 16 were slower up to
+// 8000 positions (14.2 us at 3001). Up to S positions every chunk would hold one:
+// one workgroup per kv head takes them, one position a row, and forms the sums
+// that the S records' merge would form, without records, counter or merge (1
+// position 4.8 us, 9.1 with them; 16 positions 5.5, 9.9). From there on the
+// chunks are as fast (41 positions 8.6 us, one workgroup 7.2; 201 9.3 and 9.8).
 //
 // The chunk's record (m, l, o[dim]) per head goes to the workspace; one
 // thread then bumps the kv head's counter with a device-scope (agent)
@@ -193,6 +205,9 @@ extern "C" __global__ void qmm_prefill_splitk_rope_kv(const float* __restrict__ 
 // dim = 64 * DPL (64, 128, 256); G <= GT (1, 2, 4, 8).
 namespace qmm {
 constexpr int kAttnSplits = 16;  // S
+constexpr float kLog2e = 1.44269504088896340736f;
+__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+__device__ __forceinline__ float sum4(const float (&v)[4]) { return (v[0] + v[1]) + (v[2] + v[3]); }
 
 // One lane's share of a dim-wide row in the 16-lane-row layout: lane li
 // (0..15) of every row holds dims [R * li, R * li + R) with R = dim / 16.
@@ -236,8 +251,7 @@ __device__ __forceinline__ float row16_total(float v) {
 // row i = blockIdx.y (position first + i, q row at q + i * ldq) attends to
 // positions 0 ..= first + i of the cache (which already holds them, rotated;
 // q is already rotated) and writes its normalised output to out + i * ldo.
-// The arithmetic is the S = 1 case of the chunked form (the merge of one
-// record multiplies by e^0 = 1).
+// The arithmetic is the one-chunk case.
 // PLANES (PREFILL only): instead of f32 rows, the query row's G * dim
 // outputs (whole 256-element blocks: G * dim % 256 == 0, starting at column
 // g * G * dim) go to the Q8_K GEMM planes of row blockIdx.y (q8 / d / s over
@@ -267,7 +281,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
   const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int li = lane & 15, row = 4 * wave + (lane >> 4);  // this lane's place in its row, the row's index
   const int G = heads / kv_heads;
-  constexpr int S = PREFILL ? 1 : kAttnSplits;
+  constexpr int S = kAttnSplits;
   const bool rope = !PREFILL && cos_t != nullptr;
   if constexpr (PREFILL) {
     q += blockIdx.y * ldq;
@@ -286,7 +300,10 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
   }
 
   const int n = p + 1;
-  const int L = (n + S - 1) / S;
+  const bool each = !PREFILL && n <= S;  // a position a row, all in workgroup 0
+  const int chunks = PREFILL || each ? 1 : S;
+  if (c >= chunks) return;
+  const int L = (n + chunks - 1) / chunks;
   const int j0 = min(c * L, n), j1 = min(j0 + L, n);
   const int nc = j1 - j0;
   const bool own = j0 <= p && p < j1;
@@ -321,10 +338,10 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     }
   }
 
-  float m[GT], l[GT], o[GT][R];
+  float m[GT], ml[GT], l[GT], o[GT][R];  // ml = m log2 e
 #pragma unroll
   for (int h = 0; h < GT; ++h) {
-    m[h] = -INFINITY;
+    m[h] = ml[h] = -INFINITY;
     l[h] = 0.0f;
 #pragma unroll
     for (int e = 0; e < R; ++e) o[h][e] = 0.0f;
@@ -354,7 +371,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
       for (int h = 0; h < GT; ++h) {
         float d = 0.0f;
 #pragma unroll
-        for (int e = 0; e < R; ++e) d += qv[h][e] * ks[b][e];
+        for (int e = 0; e < R; ++e) d = __builtin_fmaf(qv[h][e], ks[b][e], d);
         d = row16_total(d) * scale;
         sc[b][h] = ok ? d : -INFINITY;
       }
@@ -364,25 +381,45 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
       float mx = m[h];
 #pragma unroll
       for (int b = 0; b < B; ++b) mx = fmaxf(mx, sc[b][h]);
-      const float a = mx == -INFINITY ? 0.0f : expf(m[h] - mx);  // 0 while m = -inf
+      // e^x as 2^(x log2 e): mx log2 e is rounded once and that value is the row's
+      // maximum from here on (ml, the records and the merges), so its rounding is
+      // common to every weight
+      const float nl = mx == -INFINITY ? 0.0f : mx * kLog2e;
+      const float a = exp2_hw(ml[h] - nl);  // 0 while ml = -inf
       float ls = l[h] * a;
       float acc[R];
 #pragma unroll
       for (int e = 0; e < R; ++e) acc[e] = o[h][e] * a;
 #pragma unroll
       for (int b = 0; b < B; ++b) {
-        const float w = sc[b][h] == -INFINITY ? 0.0f : expf(sc[b][h] - mx);
+        const float w = exp2_hw(__builtin_fmaf(sc[b][h], kLog2e, -nl));
         ls += w;
 #pragma unroll
-        for (int e = 0; e < R; ++e) acc[e] += w * vs[b][e];
+        for (int e = 0; e < R; ++e) acc[e] = __builtin_fmaf(w, vs[b][e], acc[e]);
       }
       m[h] = mx;
+      ml[h] = mx == -INFINITY ? mx : nl;
       l[h] = ls;
 #pragma unroll
       for (int e = 0; e < R; ++e) o[h][e] = acc[e];
     }
   };
-  if (nwave > 0) {
+  if (each) {
+    // what scan() gives for one position: weight 1. The score is a row's of the
+    // chunk form, one rounding per operation.
+    const bool ok = row < n, at_p = rope && row == p;
+#pragma unroll
+    for (int h = 0; h < GT; ++h) {
+      float d = 0.0f;
+#pragma unroll
+      for (int e = 0; e < R; ++e) d += qv[h][e] * (at_p ? kn[e] : kr[0][e]);
+      d = row16_total(d) * scale;
+      ml[h] = ok ? fmaxf(d, -INFINITY) : -INFINITY;  // (here the score itself; scan()'s maximum of a NaN is -inf)
+      l[h] = 1.0f;
+#pragma unroll
+      for (int e = 0; e < R; ++e) o[h][e] = at_p ? vn[e] : vr[0][e];
+    }
+  } else if (nwave > 0) {
     int i0 = 0;
     for (; i0 + B < nwave; i0 += B) {
       // next batch in flight (clamped, unconditional) while this one is scored
@@ -413,26 +450,47 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
   if (li == 0) {
 #pragma unroll
     for (int h = 0; h < GT; ++h) {
-      wst[row][2 * h] = m[h];
+      wst[row][2 * h] = ml[h];
       wst[row][2 * h + 1] = l[h];
     }
   }
   __syncthreads();
+  if (each) {
+    for (int i = t; i < G * dim; i += NT) {
+      const int h = i / dim;
+      float M = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < S; ++w) M = fmaxf(M, wst[w][2 * h]);
+      float lsum = 0.0f, osum = 0.0f;
+#pragma unroll
+      for (int w = 0; w < S; ++w) {
+        if (wst[w][2 * h] != -INFINITY) {
+          const float a = expf(wst[w][2 * h] - M);
+          lsum += a;
+          osum += wo[w][i] * a;
+        }
+      }
+      out[(size_t)g * G * dim + i] = osum / lsum;
+    }
+    return;
+  }
   const size_t rec = (size_t)dim + 2;  // per (chunk, head): m, l, o[dim]
   for (int i = t; i < G * dim; i += NT) {
     const int h = i / dim, d = i % dim;
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NR; ++w) M = fmaxf(M, wst[w][2 * h]);
-    float lsum = 0.0f, osum = 0.0f;
+    // four partial sums: a shorter chain of roundings (and of instructions)
+    float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, os[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < NR; ++w) {
       if (wst[w][2 * h] != -INFINITY) {
-        const float a = expf(wst[w][2 * h] - M);
-        lsum += wst[w][2 * h + 1] * a;
-        osum += wo[w][i] * a;
+        const float a = exp2_hw(wst[w][2 * h] - M);
+        ls[w & 3] += wst[w][2 * h + 1] * a;
+        os[w & 3] += wo[w][i] * a;
       }
     }
+    const float lsum = sum4(ls), osum = sum4(os);
     if constexpr (PLANES) {
       ob[i] = osum / lsum;
       continue;
@@ -480,16 +538,16 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     float M = -INFINITY;
 #pragma unroll
     for (int cc = 0; cc < S; ++cc) M = fmaxf(M, mc[cc]);
-    float lsum = 0.0f, osum = 0.0f;
+    float lsum[4] = {0.0f, 0.0f, 0.0f, 0.0f}, osum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int cc = 0; cc < S; ++cc) {
       if (mc[cc] != -INFINITY) {
-        const float w = expf(mc[cc] - M);
-        lsum += lc[cc] * w;
-        osum += oc[cc] * w;
+        const float w = exp2_hw(mc[cc] - M);
+        lsum[cc & 3] += lc[cc] * w;
+        osum[cc & 3] += oc[cc] * w;
       }
     }
-    out[(size_t)h * dim + d] = osum / lsum;
+    out[(size_t)h * dim + d] = sum4(osum) / sum4(lsum);
   }
   if (t == 0) __hip_atomic_store(counters + g, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -69,7 +69,6 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
   constexpr int dim = 32 * DT;
   constexpr int CH = dim / 4;  // 16-byte chunks of a key row
   constexpr int HC = CH / 2;   // those of one lane half
-  constexpr float kLog2e = 1.44269504088896340736f;
   __shared__ __attribute__((aligned(16))) float buf[kPaWaves][kPaKeys * dim];  // a wave's K tile, then its O^T
   __shared__ __attribute__((aligned(16))) float qb[kPaCols * dim];             // the columns' queries
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -254,7 +253,7 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
     *reinterpret_cast<FloatN<DT>*>(kb + col * dim + DT * ((8 * (r >> 2) + 4 * half + (r & 3)) ^ col)) = o;
   }
   if (half == 0) {
-    st[wave][0][col] = m;
+    st[wave][0][col] = m == -INFINITY ? m : ml;  // in the exponentials' own units
     st[wave][1][col] = l;
   }
   if (lane == 0) sbad[wave] = bad;
@@ -304,7 +303,7 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
 #pragma unroll
     for (int w = 0; w < kPaWaves; ++w) {
       if (st[w][0][c] != -INFINITY) {
-        const float a = expf(st[w][0][c] - M);
+        const float a = __builtin_amdgcn_exp2f(st[w][0][c] - M);
         const FloatN<DT> x = *reinterpret_cast<const FloatN<DT>*>(buf[w] + c * dim + DT * (e ^ c));
         lsum += st[w][1][c] * a;
 #pragma unroll
