@@ -193,6 +193,11 @@ def _stream(device: torch.device) -> ctypes.c_void_p:
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+# The current stream's handle on a device index, without building a Stream object for it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                      lambda index: torch.cuda.current_stream(index).cuda_stream)
+
+
 class GgmlDType(enum.IntEnum):
     """GGML block types of the quantized path (GGUF numbering)."""
 
@@ -372,28 +377,43 @@ class QMatMul:
         return cls(qtensor)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        n, k = self.qtensor.shape
+        # One row is a few microseconds of kernel, so back to back the host's part sets the pace. With a device
+        # context, a Stream object and a workspace that one or two rows do not use it was 14.0 us a call; 7.6 us
+        # as here (Q4_K 1024 x 4096).
+        qt = self.qtensor
+        n, k = qt.shape
         if x.dtype != torch.float32:
             raise QmmError(1, f"QMatMul::forward expects float32 input, got {x.dtype}")
-        if x.shape[-1] != k:
-            raise QmmError(1, f"shape mismatch: input last dim {x.shape[-1]} vs weight in-dim {k}")
-        if x.device != self.qtensor.device:
-            raise QmmError(1, f"input on {x.device}, weight on {self.qtensor.device}")
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, k)
+        shape = x.shape
+        if shape[-1] != k:
+            raise QmmError(1, f"shape mismatch: input last dim {shape[-1]} vs weight in-dim {k}")
+        dev = x.device
+        if dev != qt.device:
+            raise QmmError(1, f"input on {dev}, weight on {qt.device}")
+        flat = len(shape) == 2
+        x2 = x if flat else x.reshape(-1, k)
         if x2.stride(-1) != 1:
             x2 = x2.contiguous()
         m = x2.shape[0]
-        y = torch.empty((m, n), dtype=torch.float32, device=x.device)
-        if m == 0:
-            return y.reshape(*lead, n)
-        L = lib()
-        ws_bytes = int(L.qmm_matmul_workspace_size(self.qtensor.handle, m))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-        with torch.cuda.device(x.device):
-            _check(L.qmm_matmul(self.qtensor.handle, x2.data_ptr(), m, x2.stride(0), y.data_ptr(), n,
-                                ws.data_ptr(), ws_bytes, _stream(x.device)))
-        return y.reshape(*lead, n)
+        y = torch.empty((m, n), dtype=torch.float32, device=dev)
+        if m != 0:
+            L = lib()
+            h = qt.handle
+            ws, ws_bytes, ws_ptr = None, 0, None
+            if m > 2:  # one and two rows are quantized in the GEMV's prologue
+                ws_bytes = int(L.qmm_matmul_workspace_size(h, m))
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+                ws_ptr = ws.data_ptr()
+            if torch.cuda.current_device() == dev.index:
+                status = L.qmm_matmul(h, x2.data_ptr(), m, x2.stride(0), y.data_ptr(), n, ws_ptr, ws_bytes,
+                                      _raw_stream(dev.index))
+            else:
+                with torch.cuda.device(dev):
+                    status = L.qmm_matmul(h, x2.data_ptr(), m, x2.stride(0), y.data_ptr(), n, ws_ptr, ws_bytes,
+                                          _raw_stream(dev.index))
+            if status != QMM_OK:
+                raise QmmError(status, last_error())
+        return y if flat else y.reshape(*shape[:-1], n)
 
     def forward_via_f16(self, x: torch.Tensor) -> torch.Tensor:
         """QMatMul::forward_via_f16: the weight dequantized to a dense f16 tile, x cast to f16, a dense
