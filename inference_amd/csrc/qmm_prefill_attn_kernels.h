@@ -253,7 +253,9 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
     *reinterpret_cast<FloatN<DT>*>(kb + col * dim + DT * ((8 * (r >> 2) + 4 * half + (r & 3)) ^ col)) = o;
   }
   if (half == 0) {
-    st[wave][0][col] = m == -INFINITY ? m : ml;  // in the exponentials' own units
+    // in the exponentials' own units; -inf marks a wave without weights. (A wave whose
+    // scores are all NaN has the maximum -inf too, and a sum that must not be left out.)
+    st[wave][0][col] = m == -INFINITY && l == 0.0f ? m : ml;
     st[wave][1][col] = l;
   }
   if (lane == 0) sbad[wave] = bad;

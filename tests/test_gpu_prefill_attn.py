@@ -108,6 +108,21 @@ def test_non_finite_values_reach_only_the_rows_that_see_them(monkeypatch, what, 
     assert ((tiles.double() - want).abs() <= bound)[same].all()
 
 
+@pytest.mark.parametrize("key", [32, 64, 96])
+def test_nan_key_that_is_all_a_wave_sees(monkeypatch, key):
+    """A NaN key row at the first position of the second, third or fourth key tile is the only one that the
+    tile's wave sees for that position's query: every row that sees it is NaN, on both paths, and no other."""
+    first, count, heads, kv_heads, hd = 1, 110, 8, 2, 128
+    q, kc, vc = inputs(first, count, heads, kv_heads, hd, 78)
+    want, bound = reference(q, kc, vc, first, heads, hd)
+    kc[:, key, 17] = math.nan
+    for path in ("tiles", "rows"):
+        monkeypatch.setenv("QMM_PREFILL_ATTN", path)
+        got = call(q, kc, vc, first, heads, hd)
+        assert ((got.double() - want).abs() <= bound)[: key - first].all(), path
+        assert torch.isnan(got[key - first:]).all(), path
+
+
 @pytest.mark.parametrize("m,heads,kv_heads,hd", [(127, 32, 8, 128), (9, 32, 8, 128), (33, 16, 4, 64), (24, 24, 12, 128)])
 def test_tiles_write_the_o_gemms_planes(monkeypatch, m, heads, kv_heads, hd):
     """qmm_prefill_attention_o on the tile path (which writes the o GEMM's Q8_K planes) == the two calls."""
