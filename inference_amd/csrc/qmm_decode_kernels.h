@@ -158,8 +158,7 @@ extern "C" __global__ void qmm_prefill_splitk_rope_kv(const float* __restrict__ 
 // online per row, a batch of positions at a time (m = running max,
 // l = sum exp(s - m), o = sum exp(s - m) v). The next batch's k/v rows are
 // loaded while the current batch is scored. The rows' states are combined
-// through LDS. The exponentials are 2^(s log2 e - m log2 e) with one rounding
-// each; the states and records carry m log2 e, the value that was subtracted.
+// through LDS.
 //
 // What bounds it: VALU issue (dots and weighted sums of G heads over every
 // position) up to a few thousand positions on half the CUs, above a fixed ~8 us
@@ -205,8 +204,12 @@ extern "C" __global__ void qmm_prefill_splitk_rope_kv(const float* __restrict__ 
 // dim = 64 * DPL (64, 128, 256); G <= GT (1, 2, 4, 8).
 namespace qmm {
 constexpr int kAttnSplits = 16;  // S
-constexpr float kLog2e = 1.44269504088896340736f;
-__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+// The attention's exponentials, e^(s - m) as 2^((s - m) log2 e): three instructions.
+// The difference comes first: s log2 e - m log2 e in one fma saves one of them, but
+// from |m| = 1e9 or so the rounding of m log2 e alone over- or underflows 2^x.
+__device__ __forceinline__ float exp_diff(float s, float m) {
+  return __builtin_amdgcn_exp2f((s - m) * 1.44269504088896340736f);
+}
 __device__ __forceinline__ float sum4(const float (&v)[4]) { return (v[0] + v[1]) + (v[2] + v[3]); }
 
 // One lane's share of a dim-wide row in the 16-lane-row layout: lane li
@@ -338,10 +341,10 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     }
   }
 
-  float m[GT], ml[GT], l[GT], o[GT][R];  // ml = m log2 e
+  float m[GT], l[GT], o[GT][R];
 #pragma unroll
   for (int h = 0; h < GT; ++h) {
-    m[h] = ml[h] = -INFINITY;
+    m[h] = -INFINITY;
     l[h] = 0.0f;
 #pragma unroll
     for (int e = 0; e < R; ++e) o[h][e] = 0.0f;
@@ -381,24 +384,20 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
       float mx = m[h];
 #pragma unroll
       for (int b = 0; b < B; ++b) mx = fmaxf(mx, sc[b][h]);
-      // e^x as 2^(x log2 e): mx log2 e is rounded once and that value is the row's
-      // maximum from here on (ml, the records and the merges), so its rounding is
-      // common to every weight
-      const float nl = mx == -INFINITY ? 0.0f : mx * kLog2e;
-      const float a = exp2_hw(ml[h] - nl);  // 0 while ml = -inf
+      const float ref = mx == -INFINITY ? 0.0f : mx;
+      const float a = exp_diff(m[h], ref);  // 0 while m = -inf
       float ls = l[h] * a;
       float acc[R];
 #pragma unroll
       for (int e = 0; e < R; ++e) acc[e] = o[h][e] * a;
 #pragma unroll
       for (int b = 0; b < B; ++b) {
-        const float w = exp2_hw(__builtin_fmaf(sc[b][h], kLog2e, -nl));
+        const float w = exp_diff(sc[b][h], ref);
         ls += w;
 #pragma unroll
         for (int e = 0; e < R; ++e) acc[e] = __builtin_fmaf(w, vs[b][e], acc[e]);
       }
       m[h] = mx;
-      ml[h] = mx == -INFINITY ? mx : nl;
       l[h] = ls;
 #pragma unroll
       for (int e = 0; e < R; ++e) o[h][e] = acc[e];
@@ -414,7 +413,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
 #pragma unroll
       for (int e = 0; e < R; ++e) d += qv[h][e] * (at_p ? kn[e] : kr[0][e]);
       d = row16_total(d) * scale;
-      ml[h] = ok ? fmaxf(d, -INFINITY) : -INFINITY;  // (here the score itself; scan()'s maximum of a NaN is -inf)
+      m[h] = ok ? fmaxf(d, -INFINITY) : -INFINITY;  // (scan()'s maximum of a NaN is -inf)
       l[h] = 1.0f;
 #pragma unroll
       for (int e = 0; e < R; ++e) o[h][e] = at_p ? vn[e] : vr[0][e];
@@ -442,16 +441,18 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     scan(kr, vr, i0);
   }
 
-  // the rows' states -> the chunk's record per head
+  // the rows' states -> the chunk's record per head. A row without a weight (m =
+  // -inf) is left out of the merges by zeros, which a weight of 0 keeps: a branch
+  // on m for each row and head there took 0.7 us.
 #pragma unroll
   for (int h = 0; h < GT; ++h)
 #pragma unroll
-    for (int e = 0; e < R; ++e) wo[row][h * dim + R * li + e] = o[h][e];
+    for (int e = 0; e < R; ++e) wo[row][h * dim + R * li + e] = m[h] != -INFINITY ? o[h][e] : 0.0f;
   if (li == 0) {
 #pragma unroll
     for (int h = 0; h < GT; ++h) {
-      wst[row][2 * h] = ml[h];
-      wst[row][2 * h + 1] = l[h];
+      wst[row][2 * h] = m[h];
+      wst[row][2 * h + 1] = m[h] != -INFINITY ? l[h] : 0.0f;
     }
   }
   __syncthreads();
@@ -461,14 +462,14 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
       float M = -INFINITY;
 #pragma unroll
       for (int w = 0; w < S; ++w) M = fmaxf(M, wst[w][2 * h]);
+      const float ref = M == -INFINITY ? 0.0f : M;
       float lsum = 0.0f, osum = 0.0f;
 #pragma unroll
       for (int w = 0; w < S; ++w) {
-        if (wst[w][2 * h] != -INFINITY) {
-          const float a = expf(wst[w][2 * h] - M);
-          lsum += a;
-          osum += wo[w][i] * a;
-        }
+        if (w >= __builtin_amdgcn_readfirstlane(n)) break;
+        const float a = expf(wst[w][2 * h] - ref);
+        lsum += a;
+        osum += wo[w][i] * a;
       }
       out[(size_t)g * G * dim + i] = osum / lsum;
     }
@@ -480,15 +481,14 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NR; ++w) M = fmaxf(M, wst[w][2 * h]);
+    const float ref = M == -INFINITY ? 0.0f : M;
     // four partial sums: a shorter chain of roundings (and of instructions)
     float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, os[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < NR; ++w) {
-      if (wst[w][2 * h] != -INFINITY) {
-        const float a = exp2_hw(wst[w][2 * h] - M);
-        ls[w & 3] += wst[w][2 * h + 1] * a;
-        os[w & 3] += wo[w][i] * a;
-      }
+      const float a = exp_diff(wst[w][2 * h], ref);
+      ls[w & 3] += wst[w][2 * h + 1] * a;
+      os[w & 3] += wo[w][i] * a;
     }
     const float lsum = sum4(ls), osum = sum4(os);
     if constexpr (PLANES) {
@@ -538,14 +538,13 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     float M = -INFINITY;
 #pragma unroll
     for (int cc = 0; cc < S; ++cc) M = fmaxf(M, mc[cc]);
+    const float ref = M == -INFINITY ? 0.0f : M;
     float lsum[4] = {0.0f, 0.0f, 0.0f, 0.0f}, osum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int cc = 0; cc < S; ++cc) {
-      if (mc[cc] != -INFINITY) {
-        const float w = exp2_hw(mc[cc] - M);
-        lsum[cc & 3] += lc[cc] * w;
-        osum[cc & 3] += oc[cc] * w;
-      }
+      const float w = exp_diff(mc[cc], ref);
+      lsum[cc & 3] += lc[cc] * w;
+      osum[cc & 3] += oc[cc] * w;
     }
     out[(size_t)h * dim + d] = sum4(osum) / sum4(lsum);
   }

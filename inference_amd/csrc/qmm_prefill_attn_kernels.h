@@ -139,7 +139,7 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
 #pragma unroll
   for (int j = 0; j < DT; ++j) acc[j] = (f32x16)(0.0f);
   bool bad = false;
-  float m = -INFINITY, ml = 0.0f, l = 0.0f;  // maximum, maximum * log2 e, this half's sum
+  float m = -INFINITY, ref = 0.0f, l = 0.0f;  // maximum, what is subtracted (0 while m is -inf), this half's sum
 
   // byte offset of this lane's first K chunk; chunk c is 16 c XORed in
   unsigned kread = (unsigned)(col * dim * 4) + 16u * ((unsigned)(half * HC) ^ (unsigned)(col & (CH - 1)));
@@ -193,16 +193,13 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
       mx = fmaxf(mx, s0[r]);
     }
     mx = fmaxf(m, half_max(mx));
-    const float nml = mx == -INFINITY ? 0.0f : mx * kLog2e;
-    const float a = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml - nml);
+    ref = mx == -INFINITY ? 0.0f : mx;
+    const float a = exp_diff(m, ref);  // 0 while m = -inf
     l *= a;
     m = mx;
-    ml = nml;
-    // e^(s - m) as 2^(s log2 e - m log2 e) with one rounding; the rounding of
-    // m log2 e is the same for every term of a column and cancels in o / l
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s0[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[r], kLog2e, -ml));
+      s0[r] = exp_diff(s0[r], ref);
       l += s0[r];
     }
     if (diag) {
@@ -253,9 +250,9 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
     *reinterpret_cast<FloatN<DT>*>(kb + col * dim + DT * ((8 * (r >> 2) + 4 * half + (r & 3)) ^ col)) = o;
   }
   if (half == 0) {
-    // in the exponentials' own units; -inf marks a wave without weights. (A wave whose
-    // scores are all NaN has the maximum -inf too, and a sum that must not be left out.)
-    st[wave][0][col] = m == -INFINITY && l == 0.0f ? m : ml;
+    // -inf marks a wave without weights (a wave whose scores are all NaN has the
+    // maximum -inf too, and a sum that must not be left out)
+    st[wave][0][col] = l == 0.0f ? m : ref;
     st[wave][1][col] = l;
   }
   if (lane == 0) sbad[wave] = bad;
@@ -305,7 +302,7 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
 #pragma unroll
     for (int w = 0; w < kPaWaves; ++w) {
       if (st[w][0][c] != -INFINITY) {
-        const float a = __builtin_amdgcn_exp2f(st[w][0][c] - M);
+        const float a = exp_diff(st[w][0][c], M);
         const FloatN<DT> x = *reinterpret_cast<const FloatN<DT>*>(buf[w] + c * dim + DT * (e ^ c));
         lsum += st[w][1][c] * a;
 #pragma unroll
