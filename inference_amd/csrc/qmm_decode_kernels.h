@@ -341,10 +341,14 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     }
   }
 
+  // Maximum, sum and weighted values. The maximum starts from the lowest finite value,
+  // not from -inf, which the scan would have to keep out of its differences.
+  constexpr float kNoMax = -3.402823466e38f;
   float m[GT], l[GT], o[GT][R];
+  bool on[GT];  // the row has a weight
 #pragma unroll
   for (int h = 0; h < GT; ++h) {
-    m[h] = -INFINITY;
+    m[h] = kNoMax;
     l[h] = 0.0f;
 #pragma unroll
     for (int e = 0; e < R; ++e) o[h][e] = 0.0f;
@@ -352,8 +356,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
   // One batch of B positions per row (i0 .. i0 + B - 1 of this row; those
   // past npos are clamped duplicates and are masked to score -inf, weight
   // 0): all B x GT scores first (16-lane row sums), then one online-softmax
-  // update per head. A row with no position yet keeps m = -inf, and the
-  // guards keep -inf - (-inf) out of exp.
+  // update per head. A row with no position yet keeps m = kNoMax and l = 0.
   // A masked slot (a clamped duplicate past the row's positions) may hold a
   // cache row that is not written yet (the chunk owning p reads row p before
   // this launch appends it): its score is -inf and its value row is replaced
@@ -384,15 +387,14 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
       float mx = m[h];
 #pragma unroll
       for (int b = 0; b < B; ++b) mx = fmaxf(mx, sc[b][h]);
-      const float ref = mx == -INFINITY ? 0.0f : mx;
-      const float a = exp_diff(m[h], ref);  // 0 while m = -inf
+      const float a = exp_diff(m[h], mx);
       float ls = l[h] * a;
       float acc[R];
 #pragma unroll
       for (int e = 0; e < R; ++e) acc[e] = o[h][e] * a;
 #pragma unroll
       for (int b = 0; b < B; ++b) {
-        const float w = exp_diff(sc[b][h], ref);
+        const float w = exp_diff(sc[b][h], mx);
         ls += w;
 #pragma unroll
         for (int e = 0; e < R; ++e) acc[e] = __builtin_fmaf(w, vs[b][e], acc[e]);
@@ -413,8 +415,8 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
 #pragma unroll
       for (int e = 0; e < R; ++e) d += qv[h][e] * (at_p ? kn[e] : kr[0][e]);
       d = row16_total(d) * scale;
-      m[h] = ok ? fmaxf(d, -INFINITY) : -INFINITY;  // (scan()'s maximum of a NaN is -inf)
-      l[h] = 1.0f;
+      m[h] = d;
+      on[h] = ok && d > -INFINITY;  // (a NaN score is left out, as scan()'s maximum leaves it out)
 #pragma unroll
       for (int e = 0; e < R; ++e) o[h][e] = at_p ? vn[e] : vr[0][e];
     }
@@ -429,6 +431,10 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
         attn_part<R>(kx[b], kc + (size_t)j * dim, li);
         attn_part<R>(vx[b], vc + (size_t)j * dim, li);
       }
+      // A prompt's rows, 3-4 heads: issued here, not sunk past the scores as the compiler
+      // has them (8 rows from position 2000, 32 / 8 heads of 128: 51 us against 45; with
+      // one head and 3 workgroups a CU it is the slower order, 64 against 69)
+      if constexpr (PREFILL && GT == 4) __builtin_amdgcn_sched_barrier(0);
       scan(kr, vr, i0);
 #pragma unroll
       for (int b = 0; b < B; ++b)
@@ -441,18 +447,22 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     scan(kr, vr, i0);
   }
 
-  // the rows' states -> the chunk's record per head. A row without a weight (m =
-  // -inf) is left out of the merges by zeros, which a weight of 0 keeps: a branch
-  // on m for each row and head there took 0.7 us.
+  // the rows' states -> the chunk's record per head. A row without a weight (no
+  // position, or only scores of -inf or NaN) is left out of the merges by a maximum of
+  // -inf and zeros, which keep a weight of 0: a branch on every row and head there
+  // took 0.7 us.
+#pragma unroll
+  for (int h = 0; h < GT; ++h)
+    if (!each) on[h] = m[h] != kNoMax || l[h] > 0.0f;
 #pragma unroll
   for (int h = 0; h < GT; ++h)
 #pragma unroll
-    for (int e = 0; e < R; ++e) wo[row][h * dim + R * li + e] = m[h] != -INFINITY ? o[h][e] : 0.0f;
+    for (int e = 0; e < R; ++e) wo[row][h * dim + R * li + e] = on[h] ? o[h][e] : 0.0f;
   if (li == 0) {
 #pragma unroll
     for (int h = 0; h < GT; ++h) {
-      wst[row][2 * h] = m[h];
-      wst[row][2 * h + 1] = m[h] != -INFINITY ? l[h] : 0.0f;
+      wst[row][2 * h] = on[h] ? m[h] : -INFINITY;
+      wst[row][2 * h + 1] = on[h] ? l[h] : 0.0f;
     }
   }
   __syncthreads();
@@ -466,7 +476,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
       float lsum = 0.0f, osum = 0.0f;
 #pragma unroll
       for (int w = 0; w < S; ++w) {
-        if (w >= __builtin_amdgcn_readfirstlane(n)) break;
+        if (w % 2 == 0 && w >= __builtin_amdgcn_readfirstlane(n)) break;
         const float a = expf(wst[w][2 * h] - ref);
         lsum += a;
         osum += wo[w][i] * a;
@@ -486,6 +496,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, os[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < NR; ++w) {
+      if (w % 4 == 0 && w >= __builtin_amdgcn_readfirstlane(nc)) break;  // rows from nc on have no position
       const float a = exp_diff(wst[w][2 * h], ref);
       ls[w & 3] += wst[w][2 * h + 1] * a;
       os[w & 3] += wo[w][i] * a;
