@@ -2090,20 +2090,33 @@ int qmm_rope_kv_append_n(float* q, float* k, const float* v, int64_t ldq, int64_
 }
 
 // Whether a prompt's causal attention runs on 32-column MFMA tiles
-// (qmm_prefill_attn_tile_*) or one workgroup per row (qmm_prefill_attention_*).
-// A tile's workgroup needs ~5 us per 128 positions (head_dim 128) however few of
-// its columns are used; a row's needs n times 0.02 / 0.04 / 0.075 us for 1 / 4 / 8
-// heads a kv head, and beyond two workgroups a CU rows also queue. Measured, rows
-// against tiles, us: 32 / 8 heads of 128, 64 rows from position 0 9.6 / 10.3, 128
-// rows 18.8 / 11.5, 1999 rows 1650 / 308; 64 rows from 500 42 / 32; 16 / 16 heads,
-// 128 rows 11.9 / 11.1; 32 / 4 heads, 12 rows 9.8 / 9.9, 32 rows 11.1 / 9.9, and 2
-// rows from 500 42 / 26; 8 / 2 heads of 64, 128 rows 7.6 / 8.0, 256 rows 14.2 / 11.1.
+// (qmm_prefill_attn_tile_*) or one workgroup per row (qmm_prefill_attention_*):
+// the smaller of two estimates in us, fitted to 2244 sizes (1-512 rows from
+// positions 0-2000, 1-8 heads a kv head, head_dim 64 and 128) at both forms.
+// Tiles: a workgroup's waves walk n positions in steps of 128, however few of its
+// columns are used; past ~400 workgroups the CUs hold two that share the matrix cores.
+// Rows: each CU holds ceil(rows * kv_heads / 256) workgroups, and every one adds its
+// scan of (about) the mean row's positions for its 1, 2, 3-4 or 5-8 heads; with
+// more heads a kv head the later, longer rows weigh more.
+// The estimate picks the slower form by more than 3% at 1% of the sizes (19% at
+// most). Rows against tiles, us: 32 / 8 heads of 128, 64 rows from position 0 6.4 /
+// 10.4, from 500 27.0 / 31.8, 128 rows 12.0 / 11.2 and 48.5 / 32.2, 384 rows 53 / 25;
+// 16 / 16 heads, 160 rows 12.4 / 16.3; 32 / 4 heads, 12 rows 6.4 / 10.2, 128 rows
+// 13.9 / 11.1; 8 / 1 heads of 64, 2 rows from 1000 30 / 28.
 // (QMM_PREFILL_ATTN=rows|tiles forces one for the sizes both take.)
-static bool prefill_attn_tiles(int64_t first, int64_t count, int heads, int kv_heads, int head_dim) {
+static bool prefill_attn_tiles(const Device* d, int64_t first, int64_t count, int heads, int kv_heads, int head_dim) {
   if (head_dim > 128) return false;  // 256: the tile's sums and V rows exceed the registers
   if (const char* e = env(kEnvPrefillAttn)) return strcmp(e, "rows") != 0;
-  if (heads / kv_heads > 4) return count * heads >= 512 || first + count >= 512;
-  return count * heads >= 2048;
+  const int G = heads / kv_heads, g = G <= 1 ? 0 : G <= 2 ? 1 : G <= 4 ? 2 : 3, hd = head_dim / 128;
+  static const double kRow0[2][4] = {{3.3, 3.5, 3.9, 4.3}, {3.4, 3.7, 4.4, 5.8}};                  // us
+  static const double kRow[2][4] = {{0.0052, 0.0085, 0.015, 0.0285}, {0.0097, 0.0128, 0.0205, 0.038}};  // us a position
+  static const double kTile0[2] = {4.5, 5.0}, kTile[2] = {3.1, 5.3};                               // us, us a step
+  const double per_cu = (double)((count * kv_heads + d->num_cu - 1) / d->num_cu);
+  const double pos = first + (g == 3 ? 0.7 : 0.5) * count;
+  const double rows = kRow0[hd][g] + kRow[hd][g] * pos * (per_cu + (g == 3 ? 0.0 : 0.1));
+  const double wgs = (double)kv_heads * ((count + 32 / G - 1) / (32 / G));
+  const double steps = (double)((first + count + 127) / 128);
+  return kTile0[hd] + kTile[hd] * steps * std::max(1.0, 0.6 * wgs / d->num_cu) < rows;
 }
 
 int qmm_prefill_attention(const float* q, int64_t ldq, const float* kcache, const float* vcache, int64_t first,
@@ -2125,7 +2138,7 @@ int qmm_prefill_attention(const float* q, int64_t ldq, const float* kcache, cons
   long long a = ldq, o = ldo;
   int f = (int)first, c = (int)count;
   hipFunction_t fn;
-  if (prefill_attn_tiles(first, count, heads, kv_heads, head_dim)) {
+  if (prefill_attn_tiles(d, first, count, heads, kv_heads, head_dim)) {
     snprintf(name, sizeof(name), "qmm_prefill_attn_tile_d%d", head_dim / 32);
     void* args[] = {&q, &a, &kcache, &vcache, &f, &c, &out, &o, &heads, &kv_heads, &max_seq, &scale};
     QMM_TRY(kernel(d, name, &fn));
@@ -2199,7 +2212,7 @@ int qmm_prefill_attention_o(const float* q, int64_t ldq, const float* kcache, co
   void* dd = b + pl.d;
   void* ss = b + pl.s;
   hipFunction_t fn;
-  if (prefill_attn_tiles(first, count, heads, kv_heads, head_dim)) {
+  if (prefill_attn_tiles(d, first, count, heads, kv_heads, head_dim)) {
     snprintf(name, sizeof(name), "qmm_prefill_attn_tile_planes_d%d", head_dim / 32);
     void* args[] = {&q, &a, &kcache, &vcache, &f, &c, &q8, &dd, &ss, &kq, &heads, &kv_heads, &max_seq, &scale};
     QMM_TRY(kernel(d, name, &fn));

@@ -78,6 +78,30 @@ def test_prefill_attention(monkeypatch, first, count, heads, kv_heads, hd, path)
     assert ((got.double() - want).abs() <= bound).all()
 
 
+# Sizes where one form is faster by 10% or more (microseconds, rows / tiles).
+FASTER = [("rows", 0, 64, 32, 8, 128),    # 6.4 / 10.4
+          ("rows", 0, 160, 16, 16, 128),  # 12.4 / 16.3
+          ("rows", 30, 128, 16, 16, 128),  # 11.2 / 16.0
+          ("rows", 0, 64, 32, 16, 128),   # 6.3 / 10.4
+          ("rows", 0, 8, 64, 8, 128),     # 6.2 / 10.3
+          ("rows", 500, 64, 32, 8, 128),  # 27.4 / 31.8
+          ("tiles", 500, 128, 32, 8, 128),  # 48.7 / 32.3
+          ("tiles", 0, 256, 32, 8, 128),  # 30.0 / 16.9
+          ("tiles", 0, 384, 8, 1, 64)]    # 18.6 / 14.1
+
+
+@pytest.mark.parametrize("form,first,count,heads,kv_heads,hd", FASTER)
+def test_the_faster_form_is_taken(monkeypatch, form, first, count, heads, kv_heads, hd):
+    """The two forms sum in different orders, so the bits tell which one ran."""
+    q, kc, vc = inputs(first, count, heads, kv_heads, hd, 79)
+    got = {None: call(q, kc, vc, first, heads, hd)}
+    for path in ("rows", "tiles"):
+        monkeypatch.setenv("QMM_PREFILL_ATTN", path)
+        got[path] = call(q, kc, vc, first, heads, hd)
+    assert not torch.equal(got["rows"], got["tiles"])
+    assert torch.equal(got[None], got[form])
+
+
 @pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
 @pytest.mark.parametrize("what", ["q", "k", "v"])
 def test_non_finite_values_reach_only_the_rows_that_see_them(monkeypatch, what, value):
