@@ -436,10 +436,16 @@ int qmm_qtensor_dequantize_to(const qmm_qtensor* t, void* dst, int out_dtype, vo
   const void* a0 = t->data;
   void* a1 = dst;
   int f = fmt;
-  void* args[] = {&a0, &a1, &nblocks, &f};
-  // a thread forms 16 bytes of outputs in each of kDqUnits (4) units
+  // A thread forms 16 bytes of outputs in each of kDqUnits (4) units, whose loads fly
+  // together; up to 8 workgroups a CU one unit each, so that a small weight spreads over
+  // the CUs (Q4_K to bf16, 4 units / 1: 256 x 256 3.1 / 2.3 us, 1024 x 4096 4.8 / 4.0;
+  // Q8_0, 4096 x 4096 8.7 / 9.2).
   const long long units = t->n * t->k * (out_dtype == QMM_F32 ? 4 : 2) / 16;
-  return launch(d, name, ceil_div(units, 4 * 256), 256, 0, (hipStream_t)stream, args);
+  const bool u1 = units <= (long long)d->num_cu * 8 * 256;
+  char kname[32];
+  snprintf(kname, sizeof(kname), "%s%s", name, u1 ? "_u1" : "");
+  void* args[] = {&a0, &a1, &nblocks, &f};
+  return launch(d, kname, ceil_div(units, u1 ? 256 : 4 * 256), 256, 0, (hipStream_t)stream, args);
 }
 
 int qmm_qtensor_dequantize(const qmm_qtensor* t, float* dst, void* stream) {

@@ -555,10 +555,10 @@ extern "C" __global__ void qmm_dev_to_ggml(const uint8_t* __restrict__ src, uint
 //
 // Bound by memory: a thread forms 16 bytes of consecutive outputs (4 f32 or 8
 // 16-bit values, always inside one sub-block), so that a wave's loads and stores
-// are whole lines, and kDqUnits of them 256 threads apart, so that their loads
-// are in flight together. 14336 x 4096 Q8_0 to f32 (295 MB) took 93 us with one
-// thread per 32 consecutive values, 128 bytes from its neighbour's, and its
-// conversion to bf16 63 us; to bf16 at once (180 MB) it takes 29 us.
+// are whole lines, and in large tensors kDqUnits of them 256 threads apart, so
+// that their loads are in flight together. 14336 x 4096 Q8_0 to f32 (295 MB) took
+// 93 us with one thread per 32 consecutive values, 128 bytes from its neighbour's,
+// and its conversion to bf16 63 us; to bf16 at once (180 MB) it takes 29 us.
 namespace qmm {
 constexpr int kDqUnits = 4;
 
@@ -673,17 +673,18 @@ struct DqUnit {
   }
 };
 
-template <int FMT, class T>
+// U units a thread, 256 threads apart.
+template <int FMT, int U, class T>
 __device__ __forceinline__ void dequantize_units(const uint8_t* __restrict__ src, T* __restrict__ y, long long nblocks) {
   constexpr int N = 16 / (int)sizeof(T);
   const long long units = nblocks * ((FMT == kFmtQ80 ? 32 : 256) / N);
-  const long long u0 = (long long)blockIdx.x * (256 * kDqUnits) + threadIdx.x;
+  const long long u0 = (long long)blockIdx.x * (256 * U) + threadIdx.x;
   const bool aligned = (reinterpret_cast<uintptr_t>(y) & 15) == 0;
-  DqUnit<FMT, N> unit[kDqUnits];
+  DqUnit<FMT, N> unit[U];
 #pragma unroll
-  for (int i = 0; i < kDqUnits; ++i) unit[i].load(src, min(u0 + 256 * i, units - 1), nblocks);
+  for (int i = 0; i < U; ++i) unit[i].load(src, min(u0 + 256 * i, units - 1), nblocks);
 #pragma unroll
-  for (int i = 0; i < kDqUnits; ++i) {
+  for (int i = 0; i < U; ++i) {
     const long long u = u0 + 256 * i;
     if (u >= units) return;
     float v[N];
@@ -697,26 +698,23 @@ __device__ __forceinline__ void dequantize_units(const uint8_t* __restrict__ src
   }
 }
 
-template <class T>
+template <int U, class T>
 __device__ __forceinline__ void dequantize_blocks(const uint8_t* __restrict__ src, T* __restrict__ y,
                                                   long long nblocks, int fmt) {
-  if (fmt == kFmtQ80) return dequantize_units<kFmtQ80>(src, y, nblocks);
-  if (fmt == kFmtQ4K) return dequantize_units<kFmtQ4K>(src, y, nblocks);
-  dequantize_units<kFmtQ6K>(src, y, nblocks);
+  if (fmt == kFmtQ80) return dequantize_units<kFmtQ80, U>(src, y, nblocks);
+  if (fmt == kFmtQ4K) return dequantize_units<kFmtQ4K, U>(src, y, nblocks);
+  dequantize_units<kFmtQ6K, U>(src, y, nblocks);
 }
 }  // namespace qmm
 
-extern "C" __global__ void __launch_bounds__(256) qmm_dequantize(const uint8_t* __restrict__ src,
-                                                                 float* __restrict__ y, long long nblocks, int fmt) {
-  qmm::dequantize_blocks(src, y, nblocks, fmt);
-}
-extern "C" __global__ void __launch_bounds__(256) qmm_dequantize_f16(const uint8_t* __restrict__ src,
-                                                                     _Float16* __restrict__ y, long long nblocks,
-                                                                     int fmt) {
-  qmm::dequantize_blocks(src, y, nblocks, fmt);
-}
-extern "C" __global__ void __launch_bounds__(256) qmm_dequantize_bf16(const uint8_t* __restrict__ src,
-                                                                      uint16_t* __restrict__ y, long long nblocks,
-                                                                      int fmt) {
-  qmm::dequantize_blocks(src, y, nblocks, fmt);
-}
+#define QMM_DEQUANTIZE(SUFFIX, T, U)                                                                              \
+  extern "C" __global__ void __launch_bounds__(256) qmm_dequantize##SUFFIX(                                       \
+      const uint8_t* __restrict__ src, T* __restrict__ y, long long nblocks, int fmt) {                           \
+    qmm::dequantize_blocks<U>(src, y, nblocks, fmt);                                                              \
+  }
+QMM_DEQUANTIZE(, float, qmm::kDqUnits)
+QMM_DEQUANTIZE(_f16, _Float16, qmm::kDqUnits)
+QMM_DEQUANTIZE(_bf16, uint16_t, qmm::kDqUnits)
+QMM_DEQUANTIZE(_u1, float, 1)
+QMM_DEQUANTIZE(_f16_u1, _Float16, 1)
+QMM_DEQUANTIZE(_bf16_u1, uint16_t, 1)

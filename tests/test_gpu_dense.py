@@ -139,3 +139,42 @@ def test_dequantize_part_filled_and_unaligned(dt, n, k):
                                                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
             np.testing.assert_array_equal(buf[off:off + n * k].view(bits).cpu().numpy(), want)
             assert (buf[:off] == 7.0).all() and (buf[off + n * k:] == 7.0).all()
+
+
+@pytest.mark.parametrize("dt", [GgmlDType.Q8_0, GgmlDType.Q4K, GgmlDType.Q6K])
+def test_dequantize_several_units_a_thread(dt):
+    """Past 8 workgroups a CU a thread forms four units (256 CUs: 2.1M f32, 4.2M 16-bit values): the last
+    workgroup part-filled, the destination on and off the 16-byte grid."""
+    import ctypes
+
+    from inference_amd import qmm
+    n, k = 16405, 256
+    wq = orc.quantize(ORC[dt], (np.random.default_rng(41).standard_normal((n, k)) * 0.02).astype(np.float32))
+    qt = QTensor.from_ggml(wq, dt, (n, k), device=DEV)
+    ref = orc.dequantize(ORC[dt], wq, n * k).astype(np.float32)
+    for tag, tdt, bits, want in ((0, torch.float32, torch.int32, ref.view(np.int32)),
+                                 (1, torch.float16, torch.int16, ref.astype(np.float16).view(np.int16)),
+                                 (30, torch.bfloat16, torch.int16, bf16_rne(ref).view(np.int16))):
+        for off in (0, 1):
+            buf = torch.full((n * k + 16,), 7.0, dtype=tdt, device=DEV)
+            qmm._check(qmm.lib().qmm_qtensor_dequantize_to(qt.handle, buf.data_ptr() + off * buf.element_size(), tag,
+                                                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+            np.testing.assert_array_equal(buf[off:off + n * k].view(bits).cpu().numpy(), want)
+            assert (buf[:off] == 7.0).all() and (buf[off + n * k:] == 7.0).all()
+
+
+@pytest.mark.parametrize("dt,at", [(GgmlDType.Q8_0, 0), (GgmlDType.Q4K, 0), (GgmlDType.Q4K, 2), (GgmlDType.Q6K, 208)])
+@pytest.mark.parametrize("scale", [0x7C00, 0xFC00, 0x7E00, 0x0001])
+def test_dequantize_bf16_of_special_scales(dt, at, scale):
+    """A block whose f16 scale is infinite, NaN or the smallest denormal: bf16 is the rounded f32 value, bit for
+    bit, and a NaN is the one that torch's conversion gives."""
+    n, k = 4, 256
+    size = {GgmlDType.Q8_0: 34, GgmlDType.Q4K: 144, GgmlDType.Q6K: 210}[dt]
+    wq = orc.quantize(ORC[dt], (np.random.default_rng(42).standard_normal((n, k)) * 0.02).astype(np.float32))
+    raw = np.frombuffer(bytes(wq), np.uint8).copy()
+    raw[size + at:size + at + 2] = (scale & 0xFF, scale >> 8)
+    qt = QTensor.from_ggml(raw, dt, (n, k), device=DEV)
+    f = qt.dequantize()
+    assert scale == 0x0001 or not torch.isfinite(f).all()
+    got, want = qt.dequantize(torch.bfloat16), f.to(torch.bfloat16)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
