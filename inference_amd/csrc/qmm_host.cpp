@@ -438,8 +438,8 @@ int qmm_qtensor_dequantize_to(const qmm_qtensor* t, void* dst, int out_dtype, vo
   int f = fmt;
   // A thread forms 16 bytes of outputs in each of kDqUnits (4) units, whose loads fly
   // together; up to 8 workgroups a CU one unit each, so that a small weight spreads over
-  // the CUs (Q4_K to bf16, 4 units / 1: 256 x 256 3.1 / 2.3 us, 1024 x 4096 4.8 / 4.0;
-  // Q8_0, 4096 x 4096 8.7 / 9.2).
+  // the CUs (Q4_K to bf16, 4 units / 1: 256 x 256 3.3 / 2.3 us, 1024 x 4096 5.1 / 4.5;
+  // Q8_0 to f16, 4096 x 4096 8.8 / 9.2).
   const long long units = t->n * t->k * (out_dtype == QMM_F32 ? 4 : 2) / 16;
   const bool u1 = units <= (long long)d->num_cu * 8 * 256;
   char kname[32];
@@ -2109,9 +2109,11 @@ int qmm_rope_kv_append_n(float* q, float* k, const float* v, int64_t ldq, int64_
 // 10.4, from 500 27.0 / 31.8, 128 rows 12.0 / 11.2 and 48.5 / 32.2, 384 rows 53 / 25;
 // 16 / 16 heads, 160 rows 12.4 / 16.3; 32 / 4 heads, 12 rows 6.4 / 10.2, 128 rows
 // 13.9 / 11.1; 8 / 1 heads of 64, 2 rows from 1000 30 / 28.
-// (QMM_PREFILL_ATTN=rows|tiles forces one for the sizes both take.)
-static bool prefill_attn_tiles(const Device* d, int64_t first, int64_t count, int heads, int kv_heads, int head_dim) {
+// (QMM_PREFILL_ATTN=rows|tiles forces one for the calls both take.)
+static bool prefill_attn_tiles(const Device* d, const float* kcache, const float* vcache, int64_t first, int64_t count,
+                               int heads, int kv_heads, int head_dim) {
   if (head_dim > 128) return false;  // 256: the tile's sums and V rows exceed the registers
+  if (((uintptr_t)kcache | (uintptr_t)vcache) % 16) return false;  // its K rows go to LDS 16 bytes a lane
   if (const char* e = env(kEnvPrefillAttn)) return strcmp(e, "rows") != 0;
   const int G = heads / kv_heads, g = G <= 1 ? 0 : G <= 2 ? 1 : G <= 4 ? 2 : 3, hd = head_dim / 128;
   static const double kRow0[2][4] = {{3.3, 3.5, 3.9, 4.3}, {3.4, 3.7, 4.4, 5.8}};                  // us
@@ -2144,7 +2146,7 @@ int qmm_prefill_attention(const float* q, int64_t ldq, const float* kcache, cons
   long long a = ldq, o = ldo;
   int f = (int)first, c = (int)count;
   hipFunction_t fn;
-  if (prefill_attn_tiles(d, first, count, heads, kv_heads, head_dim)) {
+  if (prefill_attn_tiles(d, kcache, vcache, first, count, heads, kv_heads, head_dim)) {
     snprintf(name, sizeof(name), "qmm_prefill_attn_tile_d%d", head_dim / 32);
     void* args[] = {&q, &a, &kcache, &vcache, &f, &c, &out, &o, &heads, &kv_heads, &max_seq, &scale};
     QMM_TRY(kernel(d, name, &fn));
@@ -2218,7 +2220,7 @@ int qmm_prefill_attention_o(const float* q, int64_t ldq, const float* kcache, co
   void* dd = b + pl.d;
   void* ss = b + pl.s;
   hipFunction_t fn;
-  if (prefill_attn_tiles(d, first, count, heads, kv_heads, head_dim)) {
+  if (prefill_attn_tiles(d, kcache, vcache, first, count, heads, kv_heads, head_dim)) {
     snprintf(name, sizeof(name), "qmm_prefill_attn_tile_planes_d%d", head_dim / 32);
     void* args[] = {&q, &a, &kcache, &vcache, &f, &c, &q8, &dd, &ss, &kq, &heads, &kv_heads, &max_seq, &scale};
     QMM_TRY(kernel(d, name, &fn));

@@ -102,6 +102,21 @@ def test_the_faster_form_is_taken(monkeypatch, form, first, count, heads, kv_hea
     assert torch.equal(got[None], got[form])
 
 
+@pytest.mark.parametrize("which", ["k", "v"])
+def test_caches_off_the_16_byte_grid(monkeypatch, which):
+    """A cache that starts 4 bytes past the grid runs by rows, also where tiles are asked for, with their bits."""
+    first, count, heads, kv_heads, hd = 3, 300, 8, 2, 128
+    q, kc, vc = inputs(first, count, heads, kv_heads, hd, 80)
+    monkeypatch.setenv("QMM_PREFILL_ATTN", "rows")
+    want = call(q, kc, vc, first, heads, hd)
+    monkeypatch.setenv("QMM_PREFILL_ATTN", "tiles")
+    assert not torch.equal(call(q, kc, vc, first, heads, hd), want)
+    moved = torch.empty(kc.numel() + 1, device=DEV)[1:].view(kc.shape).copy_(kc if which == "k" else vc)
+    assert moved.data_ptr() % 16 == 4
+    kc, vc = (moved, vc) if which == "k" else (kc, moved)
+    assert torch.equal(call(q, kc, vc, first, heads, hd), want)
+
+
 @pytest.mark.parametrize("value", [math.inf, -math.inf, math.nan])
 @pytest.mark.parametrize("what", ["q", "k", "v"])
 def test_non_finite_values_reach_only_the_rows_that_see_them(monkeypatch, what, value):
