@@ -110,3 +110,42 @@ def test_split_k_in_matmul_ex_accumulate(monkeypatch, norm):
         want = y0[j] + orc.matmul(orc.Q4K, xin, q.to_ggml(), k)
         assert rel_err(got[j], want) <= TOL
         assert rel_err(got[j], ref[j]) <= 1e-5
+
+
+@pytest.mark.parametrize("dt", [GgmlDType.Q4K, GgmlDType.Q8_0])
+@pytest.mark.parametrize("n", [256, 255])
+def test_split_sum_of_four_and_of_one_output_a_thread(monkeypatch, dt, n):
+    """The sum of the partials takes four outputs a thread where n, the output's row stride and its address
+    allow 16-byte accesses, and one elsewhere (an odd n, an odd stride, an output 4 bytes off the grid): the same
+    bits, nothing beside the outputs written, and the partials' sum within the roundings of three additions of
+    the f64 result."""
+    k, m, sp = 2304, 37, 3
+    qt = weight(dt, n, k, 920 + n)
+    x = torch.from_numpy(normal(921, (m, k))).to(DEV)
+    base = torch.from_numpy(normal(922, (m, n))).to(DEV)
+    monkeypatch.setenv("QMM_SPLITK", "1")
+    ref = QMatMul(qt).forward(x).double()
+    monkeypatch.setenv("QMM_SPLITK", str(sp))
+    L = qmm.lib()
+    wb = int(L.qmm_matmul_ex_workspace_size(qt.handle, m, 0))
+    ws = torch.empty(wb, dtype=torch.uint8, device=DEV)
+    scale = ref.abs().max().item()
+    for accumulate in (0, 1):
+        got = []
+        for off, ld in ((0, n), (1, n), (0, n + 1), (0, n + 4), (3, n + 7)):
+            buf = torch.full((m * ld + 8,), 7.0, device=DEV)
+            y = buf[off:off + m * ld].view(m, ld)[:, :n]
+            if accumulate:
+                y.copy_(base)
+            qmm._check(L.qmm_matmul_ex((vp * 1)(qt.handle.value), 1, x.data_ptr(), m, k, None, ctypes.c_float(0),
+                                       accumulate, (vp * 1)(y.data_ptr()), (i64 * 1)(ld), ws.data_ptr(), wb,
+                                       vp(torch.cuda.current_stream().cuda_stream)))
+            got.append(y.clone())
+            y.fill_(7.0)
+            assert (buf == 7.0).all(), (off, ld)
+        assert all(torch.equal(got[0], g) for g in got[1:])
+        want = ref + base.double() if accumulate else ref
+        # each output is k / 32 (Q8_0) or k / 256 block products (two roundings each) summed in f32, in two
+        # groupings, the partial sums at most a few times the largest output
+        blocks = k // 32 if dt == GgmlDType.Q8_0 else k // 256
+        assert (got[0].double() - want).abs().max().item() <= 2.0 ** -24 * 2 * (blocks + sp + 1) * 4 * scale
