@@ -431,10 +431,11 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
         attn_part<R>(kx[b], kc + (size_t)j * dim, li);
         attn_part<R>(vx[b], vc + (size_t)j * dim, li);
       }
-      // A prompt's rows, 3-4 heads: issued here, not sunk past the scores as the compiler
-      // has them (8 rows from position 2000, 32 / 8 heads of 128: 51 us against 45; with
-      // one head and 3 workgroups a CU it is the slower order, 64 against 69)
-      if constexpr (PREFILL && GT == 4) __builtin_amdgcn_sched_barrier(0);
+      // A prompt's rows, 2-4 heads: issued here, not sunk past the scores as the compiler
+      // has them (32 / 8 heads of 128, 8 rows from position 2000: 51 us against 45; 32 /
+      // 16, 80 rows from 1500: 84 / 79). With one head and 3 workgroups a CU it is the
+      // slower order (64 / 69).
+      if constexpr (PREFILL && (GT == 4 || (GT == 2 && DPL == 2))) __builtin_amdgcn_sched_barrier(0);
       scan(kr, vr, i0);
 #pragma unroll
       for (int b = 0; b < B; ++b)

@@ -187,11 +187,14 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
 
     float mx = -INFINITY;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s0[r] *= scale;
-      if (diag && kPaKeys * kt + 8 * (r >> 2) + 4 * half + (r & 3) > p) s0[r] = -INFINITY;
-      mx = fmaxf(mx, s0[r]);
+    for (int r = 0; r < 16; ++r) s0[r] *= scale;
+    if (diag) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (kPaKeys * kt + 8 * (r >> 2) + 4 * half + (r & 3) > p) s0[r] = -INFINITY;
     }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s0[r]);
     mx = fmaxf(m, half_max(mx));
     ref = mx == -INFINITY ? 0.0f : mx;
     const float a = exp_diff(m, ref);  // 0 while m = -inf
