@@ -2097,18 +2097,18 @@ int qmm_rope_kv_append_n(float* q, float* k, const float* v, int64_t ldq, int64_
 
 // Whether a prompt's causal attention runs on 32-column MFMA tiles
 // (qmm_prefill_attn_tile_*) or one workgroup per row (qmm_prefill_attention_*):
-// the smaller of two estimates in us, fitted to 2244 sizes (1-512 rows from
-// positions 0-2000, 1-8 heads a kv head, head_dim 64 and 128) at both forms.
-// Tiles: a workgroup's waves walk n positions in steps of 128, however few of its
+// the smaller of two estimates in us, fitted to 3870 sizes at both forms (1-512 rows
+// from positions 0-2000, 1-8 heads a kv head, head_dim 64 and 128).
+// Tiles: a workgroup's waves walk the positions in steps of 128, however few of its
 // columns are used; past ~400 workgroups the CUs hold two that share the matrix cores.
-// Rows: each CU holds ceil(rows * kv_heads / 256) workgroups, and every one adds its
-// scan of (about) the mean row's positions for its 1, 2, 3-4 or 5-8 heads; with
-// more heads a kv head the later, longer rows weigh more.
-// The estimate picks the slower form by more than 3% at 1% of the sizes (19% at
-// most). Rows against tiles, us: 32 / 8 heads of 128, 64 rows from position 0 6.4 /
-// 10.4, from 500 27.0 / 31.8, 128 rows 12.0 / 11.2 and 48.5 / 32.2, 384 rows 53 / 25;
-// 16 / 16 heads, 160 rows 12.4 / 16.3; 32 / 4 heads, 12 rows 6.4 / 10.2, 128 rows
-// 13.9 / 11.1; 8 / 1 heads of 64, 2 rows from 1000 30 / 28.
+// Rows: each CU holds ceil(rows * kv_heads / 256) workgroups, and each of those adds
+// its scan of the positions up to about the mean row for its heads (the later rows
+// are the longer ones and run last, so that somewhat more than half of the rows count).
+// The estimates pick the slower form by more than 3% at 7 of these sizes (5% at
+// most). Rows against tiles, us: 32 / 8 heads of 128, 64 rows from position 0 6.8 /
+// 10.4, from 500 26.3 / 31.8, 128 rows 12.2 / 11.2 and 47.1 / 32.4, 384 rows 50.6 /
+// 25.4; 16 / 16 heads, 160 rows 12.4 / 16.1; 32 / 4 heads, 12 rows 6.9 / 10.2, 128
+// rows 14.6 / 11.2; 8 / 1 heads of 64, 2 rows from 1000 30 / 28.
 // (QMM_PREFILL_ATTN=rows|tiles forces one for the calls both take.)
 static bool prefill_attn_tiles(const Device* d, const float* kcache, const float* vcache, int64_t first, int64_t count,
                                int heads, int kv_heads, int head_dim) {
@@ -2116,15 +2116,17 @@ static bool prefill_attn_tiles(const Device* d, const float* kcache, const float
   if (((uintptr_t)kcache | (uintptr_t)vcache) % 16) return false;  // its K rows go to LDS 16 bytes a lane
   if (const char* e = env(kEnvPrefillAttn)) return strcmp(e, "rows") != 0;
   const int G = heads / kv_heads, g = G <= 1 ? 0 : G <= 2 ? 1 : G <= 4 ? 2 : 3, hd = head_dim / 128;
-  static const double kRow0[2][4] = {{3.3, 3.5, 3.9, 4.3}, {3.4, 3.7, 4.4, 5.8}};                  // us
-  static const double kRow[2][4] = {{0.0052, 0.0085, 0.015, 0.0285}, {0.0097, 0.0128, 0.0205, 0.038}};  // us a position
-  static const double kTile0[2] = {4.5, 5.0}, kTile[2] = {3.1, 5.3};                               // us, us a step
+  // rows: fixed us, us a position and workgroup, the part of the rows that counts, workgroups to add
+  static const double kRow[2][4][4] = {
+      {{3.8, 0.0046, 0.56, -0.04}, {2.9, 0.0078, 0.48, -0.08}, {3.1, 0.0125, 0.68, 0.17}, {2.7, 0.0317, 0.74, -0.04}},
+      {{3.7, 0.0090, 0.57, 0.05}, {4.8, 0.0112, 0.67, -0.21}, {5.7, 0.0198, 0.54, -0.08}, {6.0, 0.0475, 0.72, -0.26}}};
+  static const double kTile[2][2] = {{4.5, 3.1}, {5.0, 5.3}};  // fixed us, us a step
+  const double* r = kRow[hd][g];
   const double per_cu = (double)((count * kv_heads + d->num_cu - 1) / d->num_cu);
-  const double pos = first + (g == 3 ? 0.7 : 0.5) * count;
-  const double rows = kRow0[hd][g] + kRow[hd][g] * pos * (per_cu + (g == 3 ? 0.0 : 0.1));
+  const double rows = r[0] + r[1] * (first + r[2] * count) * (per_cu + r[3]);
   const double wgs = (double)kv_heads * ((count + 32 / G - 1) / (32 / G));
   const double steps = (double)((first + count + 127) / 128);
-  return kTile0[hd] + kTile[hd] * steps * std::max(1.0, 0.6 * wgs / d->num_cu) < rows;
+  return kTile[hd][0] + kTile[hd][1] * steps * std::max(1.0, 0.6 * wgs / d->num_cu) < rows;
 }
 
 int qmm_prefill_attention(const float* q, int64_t ldq, const float* kcache, const float* vcache, int64_t first,

@@ -78,14 +78,15 @@ def test_prefill_attention(monkeypatch, first, count, heads, kv_heads, hd, path)
     assert ((got.double() - want).abs() <= bound).all()
 
 
-# Sizes where one form is faster by 10% or more (microseconds, rows / tiles).
+# Sizes where one form is faster by 6% or more (microseconds, rows / tiles).
 FASTER = [("rows", 0, 64, 32, 8, 128),    # 6.4 / 10.4
           ("rows", 0, 160, 16, 16, 128),  # 12.4 / 16.3
           ("rows", 30, 128, 16, 16, 128),  # 11.2 / 16.0
           ("rows", 0, 64, 32, 16, 128),   # 6.3 / 10.4
           ("rows", 0, 8, 64, 8, 128),     # 6.2 / 10.3
-          ("rows", 500, 64, 32, 8, 128),  # 27.4 / 31.8
-          ("tiles", 500, 128, 32, 8, 128),  # 48.7 / 32.3
+          ("rows", 500, 64, 32, 8, 128),  # 26.3 / 31.8
+          ("tiles", 0, 127, 32, 8, 128),  # 11.9 / 11.2
+          ("tiles", 500, 128, 32, 8, 128),  # 47.1 / 32.4
           ("tiles", 0, 256, 32, 8, 128),  # 30.0 / 16.9
           ("tiles", 0, 384, 8, 1, 64)]    # 18.6 / 14.1
 
