@@ -9,6 +9,8 @@
 // so a captured step replays unchanged for every position.
 #pragma once
 
+#include <type_traits>
+
 #include "qmm_common.h"
 #include "qmm_quant_kernels.h"
 
@@ -160,23 +162,28 @@ extern "C" __global__ void qmm_prefill_splitk_rope_kv(const float* __restrict__ 
 // loaded while the current batch is scored. The rows' states are combined
 // through LDS.
 //
-// What bounds it: VALU issue (dots and weighted sums of G heads over every
-// position) up to a few thousand positions on half the CUs, above a fixed ~8 us
-// of dependent round trips (position, rows, record, counter, records). 32 / 8
-// heads of 128 at 3001 positions 12.9 us, 17.2 with a library exponential and
-// separate multiplies and additions; 32 chunks instead of 16 were slower up to
-// 8000 positions (14.2 us at 3001). Up to S positions every chunk would hold one:
-// one workgroup per kv head takes them, one position a row, and forms the sums
-// that the S records' merge would form, without records, counter or merge (1
-// position 4.8 us, 9.1 with them; 16 positions 5.5, 9.9). From there on the
-// chunks are as fast (41 positions 8.6 us, one workgroup 7.2; 201 9.3 and 9.8).
+// What bounds it: a fixed ~8 us of dependent round trips (launch, position, rows,
+// record, counter, records), and above it VALU issue (dots and weighted sums of G
+// heads over every position) on half the CUs, ~1.4 us per 1000 positions. 32 / 8 heads
+// of 128: 17 positions 8.0 us, 3001 12.5, 8001 18.5 (8.6, 12.8 and 18.8 when the merges
+// branched on every row's maximum; 17.2 at 3001 with a library exponential and separate
+// multiplies and additions). 32 chunks instead of 16 were slower up to 8000 positions
+// (14.2 us at 3001).
+//
+// Up to S positions one workgroup per kv head takes them all, one position a row:
+// no loop, no records, no counter (1 position 4.6 us, 9.1 by chunks; 16 positions
+// 5.5, 9.9). It keeps the arithmetic of the chunks as they were when it was written:
+// separate multiplies and additions, the library's expf, one chain over the positions.
+// S is where a row would need a second position, not where the chunks overtake: a
+// one-workgroup scan of 41 positions took 7.2 us against 8.6, of 201 9.8 against 9.3.
 //
 // The chunk's record (m, l, o[dim]) per head goes to the workspace; one
 // thread then bumps the kv head's counter with a device-scope (agent)
 // atomic, and the workgroup that brings it to S is the last of its kv head:
 // it reads the S records back, forms
-// out = sum_c exp(m_c - M) o_c / sum_c exp(m_c - M) l_c (M = max_c m_c,
-// chunks in order) and resets the counter to zero, so the workspace is ready
+// out = sum_c exp(m_c - M) o_c / sum_c exp(m_c - M) l_c (M = max_c m_c, four
+// partial sums over every fourth chunk, then their sum; likewise over a
+// chunk's rows) and resets the counter to zero, so the workspace is ready
 // for the next launch.
 //
 // Ordering. Every access to the records is an agent-scope atomic (relaxed),
@@ -204,11 +211,28 @@ extern "C" __global__ void qmm_prefill_splitk_rope_kv(const float* __restrict__ 
 // dim = 64 * DPL (64, 128, 256); G <= GT (1, 2, 4, 8).
 namespace qmm {
 constexpr int kAttnSplits = 16;  // S
-// The attention's exponentials, e^(s - m) as 2^((s - m) log2 e): three instructions.
-// The difference comes first: s log2 e - m log2 e in one fma saves one of them, but
-// from |m| = 1e9 or so the rounding of m log2 e alone over- or underflows 2^x.
-__device__ __forceinline__ float exp_diff(float s, float m) {
-  return __builtin_amdgcn_exp2f((s - m) * 1.44269504088896340736f);
+constexpr float kLog2e = 1.44269504088896340736f;
+// The attention's exponentials, e^(s - m), are 2^(s log2 e - m log2 e): one fma, the
+// rounding of m log2 e common to every weight of a row. From |m| = 1e9 or so that
+// rounding alone over- or underflows 2^x, and past 2.36e38 the product is infinite,
+// so where it reaches 2^24 the difference is taken first, 2^((s - m) log2 e). Either
+// form is (s - off) log2 e - nl, and off and nl follow from m alone: states carry m.
+constexpr float kBigRef = 16777216.0f;  // 2^24
+struct AttnRef {
+  float off, nl;
+};
+__device__ __forceinline__ AttnRef attn_ref(float m) {
+  const float nl = m == -INFINITY ? 0.0f : m * kLog2e;
+  const bool big = !(fabsf(nl) < kBigRef);
+  return {big ? m : 0.0f, big ? 0.0f : nl};
+}
+__device__ __forceinline__ float score_weight(float s, const AttnRef& ref) {
+  return __builtin_amdgcn_exp2f(__builtin_fmaf(s - ref.off, kLog2e, -ref.nl));
+}
+// of a state with the maximum m (its own reference m log2 e, rounded); 0 for -inf
+__device__ __forceinline__ float state_weight(float m, const AttnRef& ref) {
+#pragma clang fp contract(off)
+  return __builtin_amdgcn_exp2f((m - ref.off) * kLog2e - ref.nl);
 }
 __device__ __forceinline__ float sum4(const float (&v)[4]) { return (v[0] + v[1]) + (v[2] + v[3]); }
 
@@ -341,14 +365,11 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     }
   }
 
-  // Maximum, sum and weighted values. The maximum starts from the lowest finite value,
-  // not from -inf, which the scan would have to keep out of its differences.
-  constexpr float kNoMax = -3.402823466e38f;
-  float m[GT], l[GT], o[GT][R];
-  bool on[GT];  // the row has a weight
+  float m[GT], ml[GT], l[GT], o[GT][R];  // ml = m log2 e
+  bool on[GT];                           // the row has a weight
 #pragma unroll
   for (int h = 0; h < GT; ++h) {
-    m[h] = kNoMax;
+    m[h] = ml[h] = -INFINITY;
     l[h] = 0.0f;
 #pragma unroll
     for (int e = 0; e < R; ++e) o[h][e] = 0.0f;
@@ -356,12 +377,13 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
   // One batch of B positions per row (i0 .. i0 + B - 1 of this row; those
   // past npos are clamped duplicates and are masked to score -inf, weight
   // 0): all B x GT scores first (16-lane row sums), then one online-softmax
-  // update per head. A row with no position yet keeps m = kNoMax and l = 0.
+  // update per head. A row with no position yet keeps m = -inf, and the
+  // guard keeps -inf - (-inf) out of the exponentials.
   // A masked slot (a clamped duplicate past the row's positions) may hold a
   // cache row that is not written yet (the chunk owning p reads row p before
   // this launch appends it): its score is -inf and its value row is replaced
   // by zeros, so nothing stale (even a NaN) reaches the sums.
-  auto scan = [&](const float (&kb)[B][R], const float (&vb)[B][R], int i0) {
+  auto scan = [&](const float (&kb)[B][R], const float (&vb)[B][R], int i0, auto any_size) {
     float sc[B][GT];
     float ks[B][R], vs[B][R];
 #pragma unroll
@@ -387,27 +409,38 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
       float mx = m[h];
 #pragma unroll
       for (int b = 0; b < B; ++b) mx = fmaxf(mx, sc[b][h]);
-      const float a = exp_diff(m[h], mx);
+      const float nl = mx == -INFINITY ? 0.0f : mx * kLog2e;
+      float a, w[B];
+      if constexpr (decltype(any_size)::value) {
+        const AttnRef ref = attn_ref(mx);
+        a = state_weight(m[h], ref);
+#pragma unroll
+        for (int b = 0; b < B; ++b) w[b] = score_weight(sc[b][h], ref);
+      } else {
+        a = __builtin_amdgcn_exp2f(ml[h] - nl);  // 0 while ml = -inf
+#pragma unroll
+        for (int b = 0; b < B; ++b) w[b] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[b][h], kLog2e, -nl));
+      }
       float ls = l[h] * a;
       float acc[R];
 #pragma unroll
       for (int e = 0; e < R; ++e) acc[e] = o[h][e] * a;
 #pragma unroll
       for (int b = 0; b < B; ++b) {
-        const float w = exp_diff(sc[b][h], mx);
-        ls += w;
+        ls += w[b];
 #pragma unroll
-        for (int e = 0; e < R; ++e) acc[e] = __builtin_fmaf(w, vs[b][e], acc[e]);
+        for (int e = 0; e < R; ++e) acc[e] = __builtin_fmaf(w[b], vs[b][e], acc[e]);
       }
       m[h] = mx;
+      ml[h] = mx == -INFINITY ? mx : nl;
       l[h] = ls;
 #pragma unroll
       for (int e = 0; e < R; ++e) o[h][e] = acc[e];
     }
   };
   if (each) {
-    // what scan() gives for one position: weight 1. The score is a row's of the
-    // chunk form, one rounding per operation.
+    // a position of its own per row, with weight 1; the score one rounding per
+    // operation (scan()'s dots are fused)
     const bool ok = row < n, at_p = rope && row == p;
 #pragma unroll
     for (int h = 0; h < GT; ++h) {
@@ -431,12 +464,11 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
         attn_part<R>(kx[b], kc + (size_t)j * dim, li);
         attn_part<R>(vx[b], vc + (size_t)j * dim, li);
       }
-      // A prompt's rows, 2-4 heads: issued here, not sunk past the scores as the compiler
-      // has them (32 / 8 heads of 128, 8 rows from position 2000: 51 us against 45; 32 /
-      // 16, 80 rows from 1500: 84 / 79). With one head and 3 workgroups a CU it is the
-      // slower order (64 / 69).
-      if constexpr (PREFILL && (GT == 4 || (GT == 2 && DPL == 2))) __builtin_amdgcn_sched_barrier(0);
-      scan(kr, vr, i0);
+      // A prompt's rows, 3-4 heads: issued here, not sunk past the scores as the compiler
+      // has them (32 / 8 heads of 128, 8 rows from position 2000: 49 us against 45). With
+      // one or two heads it is the slower order where a CU holds several workgroups.
+      if constexpr (PREFILL && (GT == 4 || (GT == 8 && DPL == 4))) __builtin_amdgcn_sched_barrier(0);
+      scan(kr, vr, i0, std::false_type{});
 #pragma unroll
       for (int b = 0; b < B; ++b)
 #pragma unroll
@@ -445,7 +477,36 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
           vr[b][e] = vx[b][e];
         }
     }
-    scan(kr, vr, i0);
+    scan(kr, vr, i0, std::false_type{});
+    // Scores too large for m log2 e (see kBigRef) end in such a maximum or, where it is
+    // not the last, in an infinity or a NaN: the wave scans its positions again.
+    bool bad = false;
+#pragma unroll
+    for (int h = 0; h < GT; ++h) {
+      float z = l[h] * 0.0f;
+#pragma unroll
+      for (int e = 0; e < R; ++e) z = __builtin_fmaf(o[h][e], 0.0f, z);
+      bad |= z != 0.0f || (m[h] != -INFINITY && !(fabsf(ml[h]) < kBigRef));
+    }
+    if (__builtin_expect(__any(bad), 0)) {
+#pragma unroll
+      for (int h = 0; h < GT; ++h) {
+        m[h] = ml[h] = -INFINITY;
+        l[h] = 0.0f;
+#pragma unroll
+        for (int e = 0; e < R; ++e) o[h][e] = 0.0f;
+      }
+#pragma unroll 1
+      for (i0 = 0; i0 < nwave; i0 += B) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+          const int j = min(j0 + row + NR * (i0 + b), jlast);
+          attn_part<R>(kr[b], kc + (size_t)j * dim, li);
+          attn_part<R>(vr[b], vc + (size_t)j * dim, li);
+        }
+        scan(kr, vr, i0, std::true_type{});
+      }
+    }
   }
 
   // the rows' states -> the chunk's record per head. A row without a weight (no
@@ -454,7 +515,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
   // took 0.7 us.
 #pragma unroll
   for (int h = 0; h < GT; ++h)
-    if (!each) on[h] = m[h] != kNoMax || l[h] > 0.0f;
+    if (!each) on[h] = m[h] != -INFINITY;
 #pragma unroll
   for (int h = 0; h < GT; ++h)
 #pragma unroll
@@ -492,13 +553,13 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < NR; ++w) M = fmaxf(M, wst[w][2 * h]);
-    const float ref = M == -INFINITY ? 0.0f : M;
+    const AttnRef ref = attn_ref(M);
     // four partial sums: a shorter chain of roundings (and of instructions)
     float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, os[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int w = 0; w < NR; ++w) {
       if (w % 4 == 0 && w >= __builtin_amdgcn_readfirstlane(nc)) break;  // rows from nc on have no position
-      const float a = exp_diff(wst[w][2 * h], ref);
+      const float a = state_weight(wst[w][2 * h], ref);
       ls[w & 3] += wst[w][2 * h + 1] * a;
       os[w & 3] += wo[w][i] * a;
     }
@@ -550,11 +611,11 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
     float M = -INFINITY;
 #pragma unroll
     for (int cc = 0; cc < S; ++cc) M = fmaxf(M, mc[cc]);
-    const float ref = M == -INFINITY ? 0.0f : M;
+    const AttnRef ref = attn_ref(M);
     float lsum[4] = {0.0f, 0.0f, 0.0f, 0.0f}, osum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int cc = 0; cc < S; ++cc) {
-      const float w = exp_diff(mc[cc], ref);
+      const float w = state_weight(mc[cc], ref);
       lsum[cc & 3] += lc[cc] * w;
       osum[cc & 3] += oc[cc] * w;
     }

@@ -139,7 +139,7 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
 #pragma unroll
   for (int j = 0; j < DT; ++j) acc[j] = (f32x16)(0.0f);
   bool bad = false;
-  float m = -INFINITY, ref = 0.0f, l = 0.0f;  // maximum, what is subtracted (0 while m is -inf), this half's sum
+  float m = -INFINITY, ml = 0.0f, l = 0.0f;  // maximum, maximum * log2 e (0 while it is -inf), this half's sum
 
   // byte offset of this lane's first K chunk; chunk c is 16 c XORed in
   unsigned kread = (unsigned)(col * dim * 4) + 16u * ((unsigned)(half * HC) ^ (unsigned)(col & (CH - 1)));
@@ -196,15 +196,25 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s0[r]);
     mx = fmaxf(m, half_max(mx));
-    ref = mx == -INFINITY ? 0.0f : mx;
-    const float a = exp_diff(m, ref);  // 0 while m = -inf
+    const float nml = mx == -INFINITY ? 0.0f : mx * kLog2e;
+    float a;
+    if (__builtin_expect(__any(!(fabsf(nml) < kBigRef)), 0)) {  // (see kBigRef)
+      const AttnRef ref = attn_ref(mx);
+      a = state_weight(m, ref);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s0[r] = score_weight(s0[r], ref);
+    } else {
+      // e^(s - m) as 2^(s log2 e - m log2 e) with one rounding; the rounding of
+      // m log2 e is the same for every term of a column and cancels in o / l
+      a = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml - nml);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s0[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[r], kLog2e, -nml));
+    }
     l *= a;
     m = mx;
+    ml = nml;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s0[r] = exp_diff(s0[r], ref);
-      l += s0[r];
-    }
+    for (int r = 0; r < 16; ++r) l += s0[r];
     if (diag) {
       // 0 * v is not 0 for an infinity or a NaN in a masked position's value
       // row: such a tile is computed again below, position by position
@@ -255,7 +265,7 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
   if (half == 0) {
     // -inf marks a wave without weights (a wave whose scores are all NaN has the
     // maximum -inf too, and a sum that must not be left out)
-    st[wave][0][col] = l == 0.0f ? m : ref;
+    st[wave][0][col] = l != 0.0f && m == -INFINITY ? 0.0f : m;
     st[wave][1][col] = l;
   }
   if (lane == 0) sbad[wave] = bad;
@@ -299,13 +309,14 @@ __device__ __forceinline__ void prefill_attention_tile(const float* __restrict__
     float M = -INFINITY, lsum = 0.0f;
 #pragma unroll
     for (int w = 0; w < kPaWaves; ++w) M = fmaxf(M, st[w][0][c]);
+    const AttnRef ref = attn_ref(M);
     FloatN<DT> o;
 #pragma unroll
     for (int j = 0; j < DT; ++j) o.v[j] = 0.0f;
 #pragma unroll
     for (int w = 0; w < kPaWaves; ++w) {
       if (st[w][0][c] != -INFINITY) {
-        const float a = exp_diff(st[w][0][c], M);
+        const float a = state_weight(st[w][0][c], ref);
         const FloatN<DT> x = *reinterpret_cast<const FloatN<DT>*>(buf[w] + c * dim + DT * (e ^ c));
         lsum += st[w][1][c] * a;
 #pragma unroll
