@@ -2104,11 +2104,11 @@ int qmm_rope_kv_append_n(float* q, float* k, const float* v, int64_t ldq, int64_
 // Rows: each CU holds ceil(rows * kv_heads / 256) workgroups, and each of those adds
 // its scan of the positions up to about the mean row for its heads (the later rows
 // are the longer ones and run last, so that somewhat more than half of the rows count).
-// The estimates pick the slower form by more than 3% at 9 of these sizes (6% at
-// most). Rows against tiles, us: 32 / 8 heads of 128, 64 rows from position 0 6.8 /
-// 10.4, from 500 26.3 / 31.8, 128 rows 12.2 / 11.2 and 47.1 / 32.4, 384 rows 50.6 /
-// 25.4; 16 / 16 heads, 160 rows 12.4 / 16.1; 32 / 4 heads, 12 rows 6.9 / 10.2, 128
-// rows 14.6 / 11.2; 8 / 1 heads of 64, 2 rows from 1000 30 / 28.
+// The estimates pick the slower form by more than 3% at 6 of these sizes (8% at
+// most). Rows against tiles, us: 32 / 8 heads of 128, 64 rows from position 0 7.3 /
+// 10.7, from 500 27.0 / 32.1, 127 rows 12.8 / 11.3, 128 rows from 500 47.8 / 32.3, 384
+// rows 54.5 / 25.5; 16 / 16 heads, 160 rows 12.7 / 16.3; 32 / 4 heads, 12 rows 7.6 /
+// 10.3, 128 rows 15.4 / 11.3; 8 / 1 heads of 64, 2 rows from 1000 30 / 28.
 // (QMM_PREFILL_ATTN=rows|tiles forces one for the calls both take.)
 static bool prefill_attn_tiles(const Device* d, const float* kcache, const float* vcache, int64_t first, int64_t count,
                                int heads, int kv_heads, int head_dim) {
@@ -2118,8 +2118,8 @@ static bool prefill_attn_tiles(const Device* d, const float* kcache, const float
   const int G = heads / kv_heads, g = G <= 1 ? 0 : G <= 2 ? 1 : G <= 4 ? 2 : 3, hd = head_dim / 128;
   // rows: fixed us, us a position and workgroup, the part of the rows that counts, workgroups to add
   static const double kRow[2][4][4] = {
-      {{3.8, 0.0046, 0.56, -0.04}, {2.9, 0.0078, 0.48, -0.08}, {3.1, 0.0125, 0.68, 0.17}, {2.7, 0.0317, 0.74, -0.04}},
-      {{3.7, 0.0087, 0.57, 0.05}, {4.8, 0.0112, 0.67, -0.21}, {5.7, 0.0198, 0.54, -0.08}, {6.0, 0.0475, 0.72, -0.26}}};
+      {{3.3, 0.0053, 0.46, 0.10}, {3.3, 0.0076, 0.61, -0.10}, {3.3, 0.0125, 0.82, 0.15}, {4.7, 0.0285, 0.95, -0.04}},
+      {{4.1, 0.0090, 0.54, 0.02}, {5.1, 0.0106, 0.67, 0.04}, {5.9, 0.0211, 0.53, -0.13}, {8.6, 0.0390, 0.68, -0.42}}};
   static const double kTile[2][2] = {{4.5, 3.1}, {5.0, 5.3}};  // fixed us, us a step
   const double* r = kRow[hd][g];
   const double per_cu = (double)((count * kv_heads + d->num_cu - 1) / d->num_cu);
