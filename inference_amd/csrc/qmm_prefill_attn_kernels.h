@@ -32,9 +32,9 @@
 // running output), so the error against 64 bits stays that of the row kernel
 // (1999 rows: 1.6e-7 against 1.7e-7 of the output's norm; with one chain of
 // each it was 2.7e-7, at 296 us). 1999 rows from position 0, 32 / 8 heads of
-// 128: 308 us = 107 TFLOP/s of the causal half, against 1642 us with one
-// workgroup per row (each of which read every K and V row for G heads and ran
-// on the VALU); 700 rows 59 us against 245. The rest of the time is the
+// 128: 304 us = 108 TFLOP/s of the causal half (309 with the mask in every tile),
+// against 1642 us with one workgroup per row (each of which read every K and V
+// row for G heads and ran on the VALU); 700 rows 59 us against 245. The rest of the time is the
 // softmax's VALU work where a SIMD's two waves meet in it, and the ramp of each
 // workgroup (~3 us of merge and first loads for ~16 tiles of ~5 us a wave).
 #pragma once
