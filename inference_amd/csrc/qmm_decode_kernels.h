@@ -512,7 +512,7 @@ __device__ __forceinline__ void decode_attention(const float* __restrict__ q, co
   // the rows' states -> the chunk's record per head. A row without a weight (no
   // position, or only scores of -inf or NaN) is left out of the merges by a maximum of
   // -inf and zeros, which keep a weight of 0: a branch on every row and head there
-  // took 0.7 us.
+  // took 0.6 us.
 #pragma unroll
   for (int h = 0; h < GT; ++h)
     if (!each) on[h] = m[h] != -INFINITY;
